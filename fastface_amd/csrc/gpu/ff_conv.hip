@@ -41,6 +41,7 @@
 #include <vector>
 
 #include "ff_conv_table.h"
+#include "ff_wavek.h"
 
 namespace {
 
@@ -70,19 +71,29 @@ struct ConvLaunch {
     int grid;
     int split;
     size_t counter_bytes, ws_bytes;   // split > 1: workspace layout
+    int wk;             // the wave-split kernel's tile (ff_wavek.h), or -1: fn
 };
 
 // ws_avail: workspace bytes the caller provides (a split > 1 variant that
-// needs more falls back to the whole-K tiling).  shared (FFK_SHARED_GPU):
-// a twin launch runs at the same time, so the large tiles are kept when the
-// two grids together reach FF_MID_MAX_WG.
-ConvLaunch choose_launch(const ConvEntry* e, long long M, size_t ws_avail, bool shared = false) {
+// needs more falls back to the whole-K tiling).  FFK_SHARED_GPU: a twin
+// launch runs at the same time, so the large tiles are kept when the two
+// grids together reach FF_MID_MAX_WG.  FFK_LATENCY: the wave-split kernel
+// wherever one of its tiles gives at most a workgroup per CU (ff_wk_pick).
+ConvLaunch choose_launch(const ConvEntry* e, long long M, size_t ws_avail, int flags) {
+    const bool shared = (flags & FFK_SHARED_GPU) != 0;
+    if ((flags & FFK_LATENCY) && e->cin % FF_KSTEP == 0) {
+        const int pad = e->ks / 2, ho = (e->hin + 2 * pad - e->ks) / e->stride + 1;
+        const int t = M * ho * ho > 0xffffffffLL ? -1
+                      : ff_wk_pick(M, e->cout, e->ks * e->ks * (e->cin / FF_KSTEP),
+                                   shared ? FF_WK_MAX_WG_SHARED : FF_WK_MAX_WG);
+        if (t >= 0) return {nullptr, "wavek", e->cout, (int)ff_wk_tiles(t, M, e->cout), 1, 0, 0, t};
+    }
     long long big = ((M + e->bm - 1) / e->bm) * (e->cout / e->bn);
-    ConvLaunch l = {e->fn, e->kind, e->bn, (int)big, 1, 0, 0};
+    ConvLaunch l = {e->fn, e->kind, e->bn, (int)big, 1, 0, 0, -1};
     if (e->mid && big * (shared ? 2 : 1) < FF_MID_MAX_WG) {
         const int mbm = e->mid_bm ? e->mid_bm : 128, mbn = e->mid_bn ? e->mid_bn : 128;
         big = ((M + mbm - 1) / mbm) * (e->cout / mbn);
-        l = {e->mid, e->mid_kind ? e->mid_kind : "staged128", mbn, (int)big, 1, 0, 0};
+        l = {e->mid, e->mid_kind ? e->mid_kind : "staged128", mbn, (int)big, 1, 0, 0, -1};
     }
     if (!e->small || big >= FF_SPLIT_MIN_WG) return l;
     // the small-tile kernels: e->split K ranges, 3 where e->split is larger,
@@ -383,8 +394,12 @@ int ffk_conv(const ffk_conv_desc* d, void* stream) {
         if (a.out_bn) as.out_bn = a.out_bn + o;
         if (a.out_i32) as.out_i32 = a.out_i32 + o;
         as.M = (int)ms;
-        const ConvLaunch l = choose_launch(e, ms, d->workspace ? d->workspace_bytes : 0,
-                                           (d->flags & FFK_SHARED_GPU) != 0);
+        const ConvLaunch l = choose_launch(e, ms, d->workspace ? d->workspace_bytes : 0, d->flags);
+        if (l.wk >= 0) {
+            const int rc = ff_wk_conv(as, d, l.wk, (hipStream_t)stream);
+            if (rc != FFK_OK) return rc;
+            continue;
+        }
         if (l.split > 1) {
             as.counters = (unsigned*)d->workspace;
             as.ws = (int32_t*)((int8_t*)d->workspace + l.counter_bytes);
@@ -423,8 +438,7 @@ int ffk_conv_s2_shortcut(const ffk_conv_desc* c, const ffk_conv_desc* s, void* s
     // one launch over the whole batch: every tensor below 2 GiB
     const long long lim = 0x7fffffffLL;
     if ((long long)c->batch * c->hin * c->win * c->cin > lim || M * c->cout > lim || M * s->cin > lim) return 0;
-    const ConvLaunch l = choose_launch(e, M, c->workspace ? c->workspace_bytes : 0,
-                                       (c->flags & FFK_SHARED_GPU) != 0);
+    const ConvLaunch l = choose_launch(e, M, c->workspace ? c->workspace_bytes : 0, c->flags);
     if (l.fn != e->fn) return 0;
     ConvArgs a = conv_args(c), b = conv_args(s);
     a.M = b.M = (int)M;
@@ -507,7 +521,7 @@ size_t ffk_conv_workspace_bytes(const ffk_conv_desc* d) {
     if (d->flags & FFK_ALGO_WINOGRAD) return 0;       // (its transformed input stays on chip)
     const long long M = conv_pixels(d);
     if (M > 0x7fffffffLL) return 0;
-    return choose_launch(e, M, (size_t)-1, (d->flags & FFK_SHARED_GPU) != 0).ws_bytes;
+    return choose_launch(e, M, (size_t)-1, d->flags).ws_bytes;
 }
 
 int ffk_conv_grid(const ffk_conv_desc* d) {
@@ -521,7 +535,7 @@ int ffk_conv_grid(const ffk_conv_desc* d) {
     if (e->cin == 3) return -1;                      // (the stem sizes its persistent grid itself)
     const long long M = conv_pixels(d);
     if (M > 0x7fffffffLL) return -1;
-    return choose_launch(e, M, d->workspace ? d->workspace_bytes : 0, (d->flags & FFK_SHARED_GPU) != 0).grid;
+    return choose_launch(e, M, d->workspace ? d->workspace_bytes : 0, d->flags).grid;
 }
 
 const char* ffk_conv_variant(const ffk_conv_desc* d) {
@@ -532,7 +546,7 @@ const char* ffk_conv_variant(const ffk_conv_desc* d) {
                        ? "generic" : nullptr;
     const long long M = conv_pixels(d);
     if (M > 0x7fffffffLL) return nullptr;
-    return choose_launch(e, M, d->workspace ? d->workspace_bytes : 0, (d->flags & FFK_SHARED_GPU) != 0).kind;
+    return choose_launch(e, M, d->workspace ? d->workspace_bytes : 0, d->flags).kind;
 }
 
 // BN second output as a table: lut[c][q + 128] = BN-requant of the int8

@@ -7,18 +7,18 @@
 // 16 B per lane per load, v_dot4 signed int8 products into exact int32), so
 // that the whole 12.8 MB weight matrix is in flight at once; the batch's
 // activation rows come from L2.  Cross-lane and then cross-wave (LDS) sums
-// give the exact dot product per face.  Larger batches use the MFMA conv
-// kernel as a 1x1 GEMM (ff_conv.hip).
+// give the exact dot product per face.  From three faces on the MFMA kernels
+// run it as a 1x1 conv (ff_conv_wavek.hip, ff_conv_fc.hip above 1024 faces).
 #include <cstring>
-#include "ff_internal.h"
 #include "ff_numerics.h"
-
-int ffk_fc_gemm_launch(const ffk_fc_desc* d, hipStream_t s);
-size_t ffk_fc_split_ws_bytes(int batch);
+#include "ff_wavek.h"
 
 namespace {
 
-constexpr int FC_MAXB = 16;   // matvec path handles up to this many faces
+constexpr int FC_MAXB = 16;          // faces per matvec launch
+constexpr int FC_WAVEK_MIN = 3;      // the wave-split kernel's faces (fc_kernel)
+constexpr int FC_WAVEK_MIN_WHOLE = 5;
+constexpr int FC_WAVEK_MAX = 1024;
 
 __device__ __forceinline__ int dot16(v4i a, v4i w, int acc) {
     acc = __builtin_amdgcn_sdot4(a.x, w.x, acc, false);
@@ -114,6 +114,28 @@ __global__ void mfma_probe_kernel(int* out) {
     }
 }
 
+// Which kernel runs a head with ws_bytes of workspace.  The matvec's time grows with the faces (5.7 us
+// at 1, 7.3 at 2, 9.8 at 4, 27 at 16: each of its 256 workgroups reads every
+// face's activations); the wave-split kernel takes 7.7 us from 1 to 32 faces
+// and 36 at 1000, where the 128x128 tiles of the compiled GEMM take 38 (64
+// at 2000, the same); that one is compiled for the IResNet head only.
+// Without the workspace the wave-split kernel runs whole K: 10.3 us up to 24
+// faces, which passes the matvec at 5.
+enum FcKernel { FC_MATVEC, FC_WAVEK, FC_GEMM };
+
+FcKernel fc_kernel(const ffk_fc_desc* d, size_t ws_bytes) {
+    const bool gemm_shape = d->n == 512 && d->k == 25088;
+    if (d->path == 1) return FC_MATVEC;
+    if (d->path == 2 && !gemm_shape) return FC_GEMM;               // (refused there)
+    if (d->path == 0 && d->batch < FC_WAVEK_MIN) return FC_MATVEC;
+    if (d->path == 0 && d->batch < FC_WAVEK_MIN_WHOLE && ff_wk_fc_plan(d->batch, d->n, d->k, ws_bytes).split == 1)
+        return FC_MATVEC;
+    if (gemm_shape && d->batch > FC_WAVEK_MAX) return FC_GEMM;
+    // its buffers hold less than 2 GiB, its vectors four outputs
+    const bool fits = (d->n & 3) == 0 && (long long)d->batch * d->k <= 0x7fffffffLL && (long long)d->n * d->k <= 0x7fffffffLL;
+    return fits ? FC_WAVEK : gemm_shape ? FC_GEMM : FC_MATVEC;
+}
+
 }  // namespace
 
 extern "C" {
@@ -140,9 +162,12 @@ int ffk_pack_fc_row(const int8_t* row, int n, int k, int r, int8_t* packed) {
 }
 
 size_t ffk_fc_workspace_bytes(const ffk_fc_desc* d) {
-    if (!d || d->batch <= 0 || d->n != 512 || d->k != 25088) return 0;
-    const int path = d->path ? d->path : (d->batch <= FC_MAXB ? 1 : 2);
-    return path == 2 ? ffk_fc_split_ws_bytes(d->batch) : 0;
+    if (!d || d->batch <= 0 || d->n <= 0 || d->k <= 0 || (d->k % FF_KSTEP) != 0) return 0;
+    switch (fc_kernel(d, (size_t)-1)) {
+    case FC_WAVEK: return ff_wk_fc_plan(d->batch, d->n, d->k, (size_t)-1).ws_bytes;
+    case FC_GEMM: return ffk_fc_split_ws_bytes(d->batch);
+    default: return 0;
+    }
 }
 
 int ffk_fc(const ffk_fc_desc* d, void* stream) {
@@ -153,12 +178,11 @@ int ffk_fc(const ffk_fc_desc* d, void* stream) {
     }
     if (d->batch == 0) return FFK_OK;
     hipStream_t s = (hipStream_t)stream;
-    int path = d->path;
-    // the MFMA GEMM is compiled for the IResNet head (25088 -> 512); any
-    // other shape takes the matvec in chunks of FC_MAXB faces at every batch
-    const bool gemm_shape = d->n == 512 && d->k == 25088;
-    if (path == 0) path = (d->batch <= FC_MAXB || !gemm_shape) ? 1 : 2;
-    if (path == 2) return ffk_fc_gemm_launch(d, s);
+    switch (fc_kernel(d, d->workspace ? d->workspace_bytes : 0)) {
+    case FC_WAVEK: return ff_wk_fc(d, s);
+    case FC_GEMM: return ffk_fc_gemm_launch(d, s);
+    default: break;
+    }
     for (int b0 = 0; b0 < d->batch; b0 += FC_MAXB) {
         const int nb = d->batch - b0 < FC_MAXB ? d->batch - b0 : FC_MAXB;
         float* out = d->out ? d->out + (size_t)b0 * d->n : nullptr;

@@ -363,7 +363,7 @@ static void step_desc(FastFace* ff, int s, int batch, int fmt, int part, size_t 
         d->flags |= FFK_ALGO_WINOGRAD;
         d->w = ff->d_weights + st->wino_off;
     }
-    if (shared) d->flags |= FFK_SHARED_GPU;
+    d->flags |= FFK_LATENCY | (shared ? FFK_SHARED_GPU : 0);     /* (each launch waits for the one before) */
     d->in_scale = st->in_scale;
     d->workspace = ff->d_ws ? (int8_t*)ff->d_ws + (size_t)part * ff->ws_part : NULL;
     d->workspace_bytes = ff->ws_part;

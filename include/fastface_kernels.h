@@ -114,6 +114,13 @@ typedef struct { const float* in; float* out; } ffk_io;
                                    the two launches' combined grid.  No
                                    reference counterpart. */
 
+#define FFK_LATENCY      0x1000 /* launch-choice hint, no effect on the values:
+                                   the launch is one of a chain in which each
+                                   waits for the one before, so a small grid
+                                   is tiled for the shortest single launch
+                                   ("wavek", ffk_conv_variant), which needs
+                                   no workspace.  No reference counterpart. */
+
 /* rows of the per-layer parameter block, each `cout` floats (device) */
 enum {
     FFK_P_WS = 0,      /* weight scale                                  */
@@ -263,7 +270,8 @@ int    ffk_conv_noalloc(const ffk_conv_desc* d, void* stream);
  * stride-2 layers as four phase images), "direct" (direct-to-LDS tiles),
  * "staged" / "staged128" (register-staged tiles), "splitk" (64x64 tiles
  * with the K reduction split over workgroups), "tile64" (64x64 tiles, whole
- * K: tiny grids), "winograd", "generic" (any other geometry); NULL when no
+ * K: tiny grids), "wavek" (FFK_LATENCY: 16x32 to 64x64 tiles with the K
+ * reduction split over the waves of a workgroup), "winograd", "generic" (any other geometry); NULL when no
  * kernel applies.  No counterpart in the reference: it lets
  * tests and benchmarks name the code path they exercise. */
 const char* ffk_conv_variant(const ffk_conv_desc* d);
@@ -326,15 +334,14 @@ typedef struct {
     float          a_scale;
     float*         out;      /* [batch][n] fp32, or NULL: io->out             */
     const ffk_io*  io;
-    int            path;     /* 0 auto (the matvec up to 16 faces, the GEMM
-                                above; a head other than 25088 -> 512 takes
-                                the matvec, 16 faces per launch), 1 matvec,
+    int            path;     /* 0 auto (the matvec for 1 and 2 faces, an MFMA
+                                GEMM above), 1 matvec (16 faces per launch),
                                 2 MFMA GEMM (25088 -> 512 only)               */
     /* Optional workspace (device memory, zero-filled once, the same rules as
      * ffk_conv_desc.workspace; one workspace can serve both): the MFMA GEMM
      * path then shares each output tile's K reduction among several
-     * workgroups, which fills the GPU at a few thousand faces.  NULL or too
-     * small: one workgroup per output tile. */
+     * workgroups, which fills the GPU at up to a few thousand faces.  NULL or
+     * too small: one workgroup per output tile. */
     void*          workspace;
     size_t         workspace_bytes;
 } ffk_fc_desc;

@@ -1,0 +1,105 @@
+"""The wave-split kernel (FFK_LATENCY convs, the FC head of 3 to 1024 faces)
+at the edges of its tiles and of its launch rules, bit for bit against the
+oracle."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+import fastface_amd as fa
+from gpu_util import params_block, run_conv, run_fc
+from test_gpu_kernels import F32, _special_params, rng
+
+pytestmark = pytest.mark.gpu
+
+# (cin, cout, k, stride, H, batch, workgroups): every tile, from one short row
+# tile to the last grid it takes, ragged last row tiles, one K step up to 72
+CASES = [
+    (512, 512, 3, 1, 7, 1, 4 * 16), (512, 512, 3, 1, 7, 5, 16 * 16),                       # 16x32
+    (64, 128, 1, 1, 28, 1, 49 * 4), (256, 512, 1, 1, 7, 5, 16 * 16),
+    (256, 256, 3, 1, 14, 5, 31 * 8), (64, 64, 3, 2, 112, 1, 98 * 2),                       # 32x32
+    (256, 256, 3, 1, 14, 8, 49 * 4), (64, 128, 3, 1, 56, 1, 98 * 2), (256, 256, 3, 2, 28, 10, 62 * 4),   # 32x64
+    (256, 256, 3, 1, 14, 11, 45 * 4), (512, 512, 3, 2, 14, 31, 32 * 8),                    # 48x64
+    (256, 256, 3, 1, 14, 17, 53 * 4), (512, 512, 3, 1, 7, 41, 32 * 8),                     # 64x64
+]
+
+
+def _desc(cin, cout, k, s, H, B, flags):
+    d = fa.ffk_conv_desc()
+    d.batch, d.cin, d.cout, d.kh, d.kw, d.stride, d.pad, d.hin, d.win = B, cin, cout, k, k, s, k // 2, H, H
+    d.flags = flags
+    return C.byref(d)
+
+
+@pytest.mark.parametrize("mode", ["raw", "all", "bn_only", "inscale"])
+@pytest.mark.parametrize("cin,cout,k,s,H,B,grid", CASES)
+def test_wavek_conv(gpu_lib, oracle, cin, cout, k, s, H, B, grid, mode):
+    lib, L = gpu_lib, fa.FFK_LATENCY
+    assert lib.ffk_conv_variant(_desc(cin, cout, k, s, H, B, L)) == b"wavek"
+    assert lib.ffk_conv_grid(_desc(cin, cout, k, s, H, B, L)) == grid
+    assert lib.ffk_conv_workspace_bytes(_desc(cin, cout, k, s, H, B, L)) == 0
+    r = rng(3100 + cin + cout + k + H + B)
+    x = r.integers(-128, 128, size=(B, H, H, cin), dtype=np.int8)
+    w = r.integers(-128, 128, size=(cout, cin, k, k), dtype=np.int8)
+    x[0] = -128                                        # the largest sums
+    w[-1] = -128
+    acc = oracle.conv_i32(x, w, s, k // 2)
+    if mode == "raw":
+        assert np.array_equal(run_conv(lib, x, w, s, k // 2, raw=True, split=False, flags=L), acc)
+        return
+    ws, bias, inv = _special_params(r, cout)           # ties, NaN, infinities, denormals
+    if mode == "inscale":
+        got, _ = run_conv(lib, x, w, s, k // 2, params=params_block(cout, ws=ws, bias=bias, inv=inv), split=False,
+                          flags=fa.FFK_EPI_BIAS | fa.FFK_EPI_INSCALE | L, in_scale=0.0173)
+        assert np.array_equal(got, oracle.fused_epilogue(acc, ws=ws, bias=bias, in_scale=0.0173, inv_pc=inv))
+        return
+    ho = acc.shape[1]
+    slope = r.uniform(0, 1.5, cout).astype(F32)
+    adds = r.uniform(1e-3, 5e-2, cout).astype(F32)
+    add = r.integers(-128, 128, size=acc.shape, dtype=np.int8)
+    bsin = r.uniform(1e-3, 5e-2, cout).astype(F32)
+    bns = r.uniform(0.5, 1.5, cout).astype(F32)
+    bno = r.normal(0, 0.05, cout).astype(F32)
+    binv = (1.0 / r.uniform(0.01, 0.1, cout)).astype(F32)
+    P = params_block(cout, ws=ws, bias=bias, inv=inv, slope=slope, adds=adds, bn_sin=bsin, bn_s=bns, bn_o=bno,
+                     bn_inv=binv)
+    flags = fa.FFK_EPI_BIAS | fa.FFK_EPI_PRELU | fa.FFK_EPI_ADD | fa.FFK_EPI_BN | L
+    exp = oracle.fused_epilogue(acc, ws=ws, bias=bias, prelu=slope, add_src=add, add_scale_pc=adds, inv_pc=inv)
+    exp_bn = oracle.bn_prelu_requant(exp, in_scale_pc=bsin, bn_scale=bns, bn_offset=bno, inv_pc=binv)
+    for x_even in ([False, True] if mode == "all" and ho % 2 == 0 else [False]):
+        got, got_bn = run_conv(lib, x, w, s, k // 2, params=P, flags=flags, add=add, want_x=mode == "all",
+                               want_bn=True, split=False, x_even=x_even)
+        if mode == "all":
+            assert np.array_equal(got, exp[:, ::2, ::2] if x_even else exp)
+        assert np.array_equal(got_bn, exp_bn)
+
+
+# batches at the ends of every tile and K split of the rule, with the
+# workspace the call asks for and without one (whole K)
+@pytest.mark.parametrize("B", [3, 4, 5, 16, 17, 64, 65, 128, 129, 256, 257, 512, 513, 1024])
+@pytest.mark.parametrize("split", [True, False])
+def test_wavek_fc(gpu_lib, oracle, B, split):
+    r = rng(3200 + B)
+    K, N = 25088, 512
+    a = r.integers(-128, 128, size=(B, K), dtype=np.int8)
+    W = r.integers(-127, 128, size=(N, K), dtype=np.int8)
+    a[0] = -128
+    W[-1] = -127
+    ws = r.uniform(1e-7, 1e-5, N).astype(F32)
+    bias = r.normal(0, 0.05, N).astype(F32)
+    got = run_fc(gpu_lib, a, W, ws, bias, a_scale=0.37, split=split)
+    for b in sorted({0, B // 2, B - 1}):
+        assert np.array_equal(got[b], oracle.fc(a[b], W, ws, bias, 0.37)), b
+
+
+@pytest.mark.parametrize("B,K,N,split", [(3, 64, 12, False), (7, 192, 500, True), (33, 4096, 512, True), (70, 1024, 40, True)])
+def test_wavek_fc_other_heads(gpu_lib, oracle, B, K, N, split):
+    """Heads of other sizes: fewer K steps than waves, columns past N."""
+    r = rng(3300 + B)
+    a = r.integers(-128, 128, size=(B, K), dtype=np.int8)
+    W = r.integers(-128, 128, size=(N, K), dtype=np.int8)
+    ws = r.uniform(1e-7, 1e-5, N).astype(F32)
+    bias = r.normal(0, 0.05, N).astype(F32)
+    got = run_fc(gpu_lib, a, W, ws, bias, split=split)
+    for b in range(B):
+        assert np.array_equal(got[b], oracle.fc(a[b], W, ws, bias)), b
