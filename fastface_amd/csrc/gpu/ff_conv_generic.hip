@@ -9,9 +9,9 @@
 // double-buffered LDS ring (conv_generic_dma_kernel); other channel counts
 // stage it through registers, in 8-byte runs or byte by byte (any channel
 // count; the 3-channel input layer quantizes fp32 faces or maps uint8 pixels
-// on the fly).  The epilogue is the general form of the tuned kernels' per
-// element (in-scale, ws, bias, residual, PReLU, round half away with the x86
-// out-of-range case), then X, its even pixels only or BN(X) through the
+// on the fly).  The epilogue is the tuned kernels' per element (in-scale,
+// ws, bias, residual, PReLU, round half away, with the x86 out-of-range case
+// unless FFK_EPI_IN_RANGE), then X, its even pixels only or BN(X) through the
 // channel's table.  No LDS reuse of the input patch: each tap's run is read
 // from L2 / HBM for every output pixel.
 #include "ff_conv_table.h"
@@ -26,6 +26,7 @@ struct GenGeom {
     int ktot;       // kh * kw * cin
     int kpad;       // ktot rounded up to whole 64-byte weight steps
     unsigned in_bytes;   // the launch's int8 input tensor (below 2 GiB)
+    int vec;             // bytes per access of the int8 outputs and the residual
 };
 
 // A thread's position k in the reduction order (kh*KW + kw)*Cin + ci: tap
@@ -116,63 +117,268 @@ __device__ __forceinline__ v4i gather_a(const ConvArgs& a, const GenGeom& g, __a
     }
 }
 
-// The general epilogue per element (the tuned kernels' general form: in-scale,
-// ws, bias, residual, PReLU, round half away with the x86 out-of-range
-// case), then X, its even pixels only or BN(X) through the channel's table,
-// stored straight from registers: lane owns column wc + 32j + lane%32 and 16
-// rows of each of the wave's MI x NJ blocks at tile (m0, n0).
-template <int MI, int NJ>
-__device__ __forceinline__ void gen_epilogue(const v16i (&acc)[MI][NJ], const ConvArgs& a, const GenGeom& g,
-                                             long long m0, int n0, int wr, int wc) {
-    const int lane = threadIdx.x & 63;
-    const int hw = g.hout * g.wout;
-    const int C = g.cout;
-    const float* P = a.params;
-    const bool raw = a.out_i32 != nullptr;
-    const bool x_even = (a.flags & FFK_OUT_X_EVEN) != 0;
+// Epilogue.  The MFMAs run with the weights as the row operand, so a lane
+// ends with one pixel (column lane%32) and, per 32-channel block, four groups
+// of four consecutive channels: group r/4 holds channels (r/4)*8 + (lane/32)*4
+// + r%4.  Each group is requantized and packed into one dword of the wave's
+// staging tile, which then leaves as 16-byte chunks of a pixel's channels.
+// (Stored straight from registers a 128x128 tile was 64 byte stores per lane
+// of 32 bytes a row, and the BN output a table gather per element: 3x3 96->96
+// @45 PReLU at 33 faces 27.4 us, now 20.1; 96->128 @35 residual+BN at 196 faces
+// 129 us, now 64.)
+
+// Channels per vector of the int8 tensors' accesses: 16, 8, 4 or 1 bytes, the
+// largest that divides the channel count and every base address.
+__device__ __forceinline__ v4i chunk_load(const int8_t* p, int left, int vec) {
+    v4i v = {0, 0, 0, 0};
+    if (vec == 16) {
+        if (left >= 16) v = *reinterpret_cast<const v4i*>(p);
+        return v;
+    }
+    if (vec == 8) {
+        typedef int v2i __attribute__((ext_vector_type(2)));
 #pragma unroll
-    for (int j = 0; j < NJ; j++) {
-        const int n = n0 + wc + j * 32 + (lane & 31);
-        if (n >= C) continue;
-        float ws = 0.0f, bias = 0.0f, inv = 0.0f, slope = 0.0f, adds = 0.0f;
-        if (!raw) {
-            ws = P[FFK_P_WS * C + n];
-            bias = P[FFK_P_BIAS * C + n];
-            inv = P[FFK_P_INV * C + n];
-            slope = P[FFK_P_SLOPE * C + n];
-            adds = P[FFK_P_ADDSCALE * C + n];
+        for (int h = 0; h < 2; h++)
+            if (left >= 8 * h + 8) {
+                const v2i u = *reinterpret_cast<const v2i*>(p + 8 * h);
+                v[2 * h] = u[0];
+                v[2 * h + 1] = u[1];
+            }
+        return v;
+    }
+    if (vec == 4) {
+#pragma unroll
+        for (int h = 0; h < 4; h++)
+            if (left >= 4 * h + 4) v[h] = *reinterpret_cast<const int*>(p + 4 * h);
+        return v;
+    }
+#pragma unroll
+    for (int e = 0; e < 16; e++)
+        if (e < left) v[e >> 2] |= (int)((uint32_t)(uint8_t)p[e] << (8 * (e & 3)));
+    return v;
+}
+
+__device__ __forceinline__ void chunk_store(int8_t* p, v4i v, int left, int vec) {
+    if (vec == 16) {
+        if (left >= 16) *reinterpret_cast<v4i*>(p) = v;
+    } else if (vec == 8) {
+        typedef int v2i __attribute__((ext_vector_type(2)));
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+            if (left >= 8 * h + 8) *reinterpret_cast<v2i*>(p + 8 * h) = v2i{v[2 * h], v[2 * h + 1]};
+    } else if (vec == 4) {
+#pragma unroll
+        for (int h = 0; h < 4; h++)
+            if (left >= 4 * h + 4) *reinterpret_cast<int*>(p + 4 * h) = v[h];
+    } else {
+#pragma unroll
+        for (int e = 0; e < 16; e++)
+            if (e < left) p[e] = (int8_t)((uint32_t)v[e >> 2] >> (8 * (e & 3)));
+    }
+}
+
+constexpr int GEN_NPRM = 5;                           // parameter rows the epilogue reads
+constexpr int gen_stage_bytes(int MI, int NJ) { return MI * 32 * (NJ * 32 + 16); }
+
+// The tile's parameter rows [GEN_NPRM][BN] -> LDS (before the K loop, whose
+// barriers make them visible)
+template <int BN>
+__device__ __forceinline__ void gen_params(const ConvArgs& a, const GenGeom& g, int n0, float* prm) {
+    if (a.out_i32) return;
+    constexpr int rows[GEN_NPRM] = {FFK_P_WS, FFK_P_BIAS, FFK_P_SLOPE, FFK_P_ADDSCALE, FFK_P_INV};
+#pragma unroll
+    for (int r = 0; r < GEN_NPRM; r++)
+        for (int c = threadIdx.x; c < BN; c += blockDim.x)
+            prm[r * BN + c] = n0 + c < g.cout ? a.params[rows[r] * g.cout + n0 + c] : 0.0f;
+}
+
+// The BN tables go through LDS 64 at a time (pitch FF_LUT_PITCH): round j
+// holds those of the j-th 32-channel block of both wave columns (all 128 of a
+// tile at once would leave two workgroups per CU instead of four: 320->192
+// 5x5 @65 at 8 faces, 530 workgroups, 187 us against 129).  A thread's four
+// 16-byte pieces of round j:
+constexpr int GEN_LUT_BYTES = 64 * FF_LUT_PITCH;
+
+template <int NJ>
+__device__ __forceinline__ void gen_lut_load(const ConvArgs& a, const GenGeom& g, int n0, int j, v4i (&t)[4]) {
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        const int i = k * 256 + threadIdx.x;
+        const int c = i >> 4, n = n0 + (c >> 5) * (NJ * 32) + j * 32 + (c & 31);
+        typedef int v4i_any __attribute__((ext_vector_type(4), aligned(1)));
+        t[k] = v4i{0, 0, 0, 0};
+        if (n < g.cout) t[k] = *reinterpret_cast<const v4i_any*>(a.bn_lut + (size_t)n * 256 + (i & 15) * 16);
+    }
+}
+
+__device__ __forceinline__ void gen_lut_store(const v4i (&t)[4], int8_t* lut) {
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        const int i = k * 256 + threadIdx.x;
+        *reinterpret_cast<v4i*>(lut + (i >> 4) * FF_LUT_PITCH + (i & 15) * 16) = t[k];
+    }
+}
+
+// The wave's MI x NJ blocks at tile (m0 + wr, n0 + wc) to the staging tile
+// `stage` and X to memory.  prm: the tile's parameter rows.
+template <int MI, int NJ, int BN, bool RNG>
+__device__ __forceinline__ void gen_epi_i8(const v16i (&acc)[MI][NJ], const ConvArgs& a, const GenGeom& g, long long m0,
+                                           int n0, int wc, int8_t* stage, const float* prm) {
+    typedef float v4f __attribute__((ext_vector_type(4)));
+    constexpr int P = NJ * 32 + 16;                    // staging row pitch
+    constexpr int CH = NJ * 2, RPI = 64 / CH;          // 16-byte chunks per row, rows per chunk access
+    const int lane = threadIdx.x & 63;
+    const int lc = lane & 31, lh = lane >> 5;
+    const bool add = (a.flags & FFK_EPI_ADD) != 0, prelu = (a.flags & FFK_EPI_PRELU) != 0;
+    const bool insc = !RNG && (a.flags & FFK_EPI_INSCALE);
+    if (add) {
+#pragma unroll
+        for (int k = 0; k < MI * 32 / RPI; k++) {
+            const int row = lane / CH + k * RPI, n = n0 + wc + (lane % CH) * 16;
+            const long long m = m0 + row;
+            v4i v = {0, 0, 0, 0};
+            if (m < a.M && n < g.cout) v = chunk_load(a.add_src + (size_t)m * g.cout + n, g.cout - n, g.vec);
+            *reinterpret_cast<v4i*>(stage + row * P + (lane % CH) * 16) = v;
         }
+        __builtin_amdgcn_wave_barrier();               // (the wave's own tile: its LDS accesses run in order)
+    }
+#pragma unroll
+    for (int j = 0; j < NJ; j++)
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const int c = j * 32 + q * 8 + lh * 4;     // first channel of the group in the wave's block
+            const float* pr = prm + wc + c;
+            const v4f ws = *reinterpret_cast<const v4f*>(pr), bias = *reinterpret_cast<const v4f*>(pr + BN);
+            const v4f inv = *reinterpret_cast<const v4f*>(pr + 4 * BN);
+            v4f slope = {0, 0, 0, 0}, adds = {0, 0, 0, 0};
+            if (prelu) slope = *reinterpret_cast<const v4f*>(pr + 2 * BN);
+            if (add) adds = *reinterpret_cast<const v4f*>(pr + 3 * BN);
+#pragma unroll
+            for (int i = 0; i < MI; i++) {
+                uint32_t* t = reinterpret_cast<uint32_t*>(stage + (i * 32 + lc) * P + c);
+                const uint32_t res = add ? *t : 0u;
+                int v[4];
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    float f = (float)acc[i][j][q * 4 + e];
+                    if (insc) f = f * a.in_scale;
+                    f = f * ws[e];
+                    f = f + bias[e];
+                    if (add) f = ff::add_residual(f, (int32_t)(int8_t)(res >> (8 * e)), adds[e]);
+                    if (prelu) f = ff::prelu(f, slope[e]);
+                    v[e] = RNG ? ff::requant_haz_in_range(f * inv[e]) : ff::requant_haz(f * inv[e]);
+                }
+                const uint32_t lo = __builtin_amdgcn_perm((uint32_t)v[1], (uint32_t)v[0], 0x0c0c0400u);
+                const uint32_t hi = __builtin_amdgcn_perm((uint32_t)v[3], (uint32_t)v[2], 0x0c0c0400u);
+                *t = __builtin_amdgcn_perm(hi, lo, 0x05040100u);
+            }
+            asm volatile("" ::: "memory");             // one group at a time: bounds the live parameters
+        }
+    __builtin_amdgcn_wave_barrier();
+    const bool x_even = (a.flags & FFK_OUT_X_EVEN) != 0;
+    if (!a.out) return;
+#pragma unroll
+    for (int k = 0; k < MI * 32 / RPI; k++) {
+        const int row = lane / CH + k * RPI, ch = (lane % CH) * 16, n = n0 + wc + ch;
+        const long long m = m0 + row;
+        if (m >= a.M || n >= g.cout) continue;
+        const v4i v = *reinterpret_cast<const v4i*>(stage + row * P + ch);
+        const size_t o = (size_t)m * g.cout + n;
+        if (!x_even) {
+            chunk_store(a.out + o, v, g.cout - n, g.vec);
+        } else {
+            const int hw = g.hout * g.wout;
+            const int bb = (int)(m / hw);
+            const int rem = (int)(m - (long long)bb * hw);
+            const int oh = rem / g.wout, ow = rem - oh * g.wout;
+            if (!((oh | ow) & 1))
+                chunk_store(a.out + (((size_t)bb * (g.hout / 2) + (oh >> 1)) * (g.wout / 2) + (ow >> 1)) * g.cout + n, v,
+                            g.cout - n, g.vec);
+        }
+    }
+}
+
+// BN(X) of the staging tile's j-th 32-channel block, through the round's
+// tables (those of this wave's column at `lut`)
+template <int MI, int NJ>
+__device__ __forceinline__ void gen_bn_round(const ConvArgs& a, const GenGeom& g, long long m0, int n0, int j,
+                                             const int8_t* stage, const int8_t* lut) {
+    const int lane = threadIdx.x & 63;
+    const int ch = (lane & 1) * 16, n = n0 + j * 32 + ch;
+#pragma unroll
+    for (int i = 0; i < MI; i++) {
+        const int row = i * 32 + (lane >> 1);
+        const long long m = m0 + row;
+        if (m >= a.M || n >= g.cout) continue;
+        const v4i v = *reinterpret_cast<const v4i*>(stage + row * (NJ * 32 + 16) + j * 32 + ch);
+        const int8_t* L = lut + ch * FF_LUT_PITCH + 128;
+        v4i w;
+#pragma unroll
+        for (int d = 0; d < 4; d++) {
+            uint32_t b[4];
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                b[e] = (uint8_t)L[(d * 4 + e) * FF_LUT_PITCH + (int8_t)((uint32_t)v[d] >> (8 * e))];
+            const uint32_t lo = __builtin_amdgcn_perm(b[1], b[0], 0x0c0c0400u);
+            const uint32_t hi = __builtin_amdgcn_perm(b[3], b[2], 0x0c0c0400u);
+            w[d] = (int)__builtin_amdgcn_perm(hi, lo, 0x05040100u);
+        }
+        chunk_store(a.out_bn + (size_t)m * g.cout + n, w, g.cout - n, g.vec);
+    }
+}
+
+// All of it after the K loop: smem is the workgroup's LDS (the operands are
+// consumed), gen_epi_bytes of it.
+constexpr int gen_epi_bytes(int BM, int BN, bool LUT) {
+    return 4 * gen_stage_bytes(BM / 64, BN / 64) + (LUT ? GEN_LUT_BYTES : 0);
+}
+
+template <int BM, int BN, bool LUT>
+__device__ __forceinline__ void gen_epilogue(const v16i (&acc)[BM / 64][BN / 64], const ConvArgs& a, const GenGeom& g,
+                                             long long m0, int n0, int wr, int wc, int8_t* smem, const float* prm) {
+    constexpr int MI = BM / 64, NJ = BN / 64;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    if (a.out_i32) {
 #pragma unroll
         for (int i = 0; i < MI; i++)
 #pragma unroll
-            for (int e = 0; e < 16; e++) {
-                const long long mm = m0 + wr + i * 32 + (e >> 2) * 8 + (lane >> 5) * 4 + (e & 3);
-                if (mm >= a.M) continue;
-                const size_t o = (size_t)mm * C + n;
-                if (raw) {
-                    a.out_i32[o] = acc[i][j][e];
-                    continue;
-                }
-                float f = (float)acc[i][j][e];
-                if (a.flags & FFK_EPI_INSCALE) f = f * a.in_scale;
-                f = f * ws;
-                f = f + bias;
-                if (a.flags & FFK_EPI_ADD) f = ff::add_residual(f, (int32_t)a.add_src[o], adds);
-                if (a.flags & FFK_EPI_PRELU) f = ff::prelu(f, slope);
-                const int q = ff::requant_haz(f * inv);
-                if (a.out) {
-                    if (!x_even) {
-                        a.out[o] = (int8_t)q;
+            for (int j = 0; j < NJ; j++)
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    const long long m = m0 + wr + i * 32 + (lane & 31);
+                    const int n = n0 + wc + j * 32 + q * 8 + (lane >> 5) * 4;
+                    if (m >= a.M) continue;
+                    typedef int v4i_any __attribute__((ext_vector_type(4), aligned(4)));
+                    int32_t* o = a.out_i32 + (size_t)m * g.cout + n;
+                    if (n + 3 < g.cout) {
+                        *reinterpret_cast<v4i_any*>(o) = v4i{acc[i][j][q * 4], acc[i][j][q * 4 + 1], acc[i][j][q * 4 + 2],
+                                                             acc[i][j][q * 4 + 3]};
                     } else {
-                        const int bb = (int)(mm / hw);
-                        const int rem = (int)(mm - (long long)bb * hw);
-                        const int oh = rem / g.wout, ow = rem - oh * g.wout;
-                        if (!((oh | ow) & 1))
-                            a.out[(((size_t)bb * (g.hout / 2) + (oh >> 1)) * (g.wout / 2) + (ow >> 1)) * C + n] = (int8_t)q;
+#pragma unroll
+                        for (int e = 0; e < 3; e++)
+                            if (n + e < g.cout) o[e] = acc[i][j][q * 4 + e];
                     }
                 }
-                if (a.flags & FFK_EPI_BN) a.out_bn[o] = a.bn_lut[n * 256 + q + 128];
-            }
+        return;
+    }
+    int8_t* lut = smem + 4 * gen_stage_bytes(MI, NJ);
+    int8_t* stage = smem + wave * gen_stage_bytes(MI, NJ);
+    v4i t[4];
+    if constexpr (LUT) gen_lut_load<NJ>(a, g, n0, 0, t);
+    __syncthreads();                                   // every wave is done with the operands
+    if ((a.flags & FFK_EPI_IN_RANGE) && !(a.flags & FFK_EPI_INSCALE))
+        gen_epi_i8<MI, NJ, BN, true>(acc, a, g, m0 + wr, n0, wc, stage, prm);
+    else
+        gen_epi_i8<MI, NJ, BN, false>(acc, a, g, m0 + wr, n0, wc, stage, prm);
+    if constexpr (LUT) {
+#pragma unroll
+        for (int j = 0; j < NJ; j++) {
+            if (j) __syncthreads();                    // the last round's tables are read
+            gen_lut_store(t, lut);
+            if (j + 1 < NJ) gen_lut_load<NJ>(a, g, n0, j + 1, t);
+            __syncthreads();
+            gen_bn_round<MI, NJ>(a, g, m0 + wr, n0 + wc, j, stage, lut + (wc / (NJ * 32)) * 32 * FF_LUT_PITCH);
+        }
     }
 }
 
@@ -184,7 +390,7 @@ __device__ __forceinline__ void gen_epilogue(const v16i (&acc)[MI][NJ], const Co
 // are in flight meanwhile.  A 128-wide tile halves the gathers of the other
 // operand per MAC: every staged A row serves BN output channels, every B row
 // BM output pixels.
-template <int RUN, int BM, int BN>
+template <int RUN, int BM, int BN, bool LUT>
 __global__ __launch_bounds__(256) void conv_generic_kernel(ConvArgs a, GenGeom g) {
     constexpr int AR = BM / 64, BR = BN / 64;          // operand rows each thread stages
     constexpr int MI = BM / 64, NJ = BN / 64;          // 32x32 blocks per wave (2 x 2 waves)
@@ -192,8 +398,11 @@ __global__ __launch_bounds__(256) void conv_generic_kernel(ConvArgs a, GenGeom g
     // at once, their loads in flight together, measured 7-48 % slower:
     // fewer waves per SIMD, the gathers' VALU work back to back)
     constexpr int PITCH = 80;                          // LDS row pitch of the staged operands
-    __shared__ __align__(16) int8_t As[BM * PITCH];
-    __shared__ __align__(16) int8_t Bs[BN * PITCH];
+    constexpr int LDS_K = (BM + BN) * PITCH, LDS_E = gen_epi_bytes(BM, BN, LUT);
+    __shared__ __align__(16) int8_t smem[LDS_K > LDS_E ? LDS_K : LDS_E];
+    __shared__ __align__(16) float prm[GEN_NPRM * BN];
+    int8_t* As = smem;
+    int8_t* Bs = smem + BM * PITCH;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int tiles_n = (g.cout + BN - 1) / BN;
     // Workgroups go round-robin over the 8 XCDs: give each XCD a contiguous
@@ -246,6 +455,7 @@ __global__ __launch_bounds__(256) void conv_generic_kernel(ConvArgs a, GenGeom g
     for (int i = 0; i < AR; i++) ra[i] = gather_a<RUN>(a, g, r_in, x, mrow[i], base[i], ih0[i], iw0[i], cur);
 #pragma unroll
     for (int i = 0; i < BR; i++) rb[i] = load_b(0, i);
+    gen_params<BN>(a, g, n0, prm);
     for (int k0 = 0; k0 < g.kpad; k0 += 64) {
         __syncthreads();                                  // the previous step's fragments are read
 #pragma unroll
@@ -272,11 +482,11 @@ __global__ __launch_bounds__(256) void conv_generic_kernel(ConvArgs a, GenGeom g
 #pragma unroll
             for (int i = 0; i < MI; i++)
 #pragma unroll
-                for (int j = 0; j < NJ; j++) acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(A[i], B[j], acc[i][j], 0, 0, 0);
+                for (int j = 0; j < NJ; j++) acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(B[j], A[i], acc[i][j], 0, 0, 0);
         }
     }
 
-    gen_epilogue<MI, NJ>(acc, a, g, m0, n0, wr, wc);
+    gen_epilogue<BM, BN, LUT>(acc, a, g, m0, n0, wr, wc, smem, prm);
 }
 
 // Cin % 16 == 0 (16-byte channel runs): the same tiles with the operands
@@ -293,14 +503,16 @@ __global__ __launch_bounds__(256) void conv_generic_kernel(ConvArgs a, GenGeom g
 // out-of-range offset.
 constexpr int GEN_NST = 2;
 
-template <int BM, int BN>
+template <int BM, int BN, bool LUT>
 __global__ __launch_bounds__(256, 2) void conv_generic_dma_kernel(ConvArgs a, GenGeom g) {
     constexpr int MI = BM / 64, NJ = BN / 64;          // 32x32 blocks per wave (2 x 2 waves)
     constexpr int A_BYTES = BM * 64, B_BYTES = BN * 64, STAGE = A_BYTES + B_BYTES;
     constexpr int A_LD = A_BYTES / (256 * 16), B_LD = B_BYTES / (256 * 16);
     constexpr int LPS = A_LD + B_LD;                   // loads per thread and stage
     static_assert((GEN_NST - 2) * LPS < 64, "vmcnt range");
-    __shared__ __align__(1024) int8_t smem[GEN_NST * STAGE];
+    constexpr int LDS_K = GEN_NST * STAGE, LDS_E = gen_epi_bytes(BM, BN, LUT);
+    __shared__ __align__(1024) int8_t smem[LDS_K > LDS_E ? LDS_K : LDS_E];
+    __shared__ __align__(16) float prm[GEN_NPRM * BN];
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lane = tid & 63;
@@ -371,6 +583,7 @@ __global__ __launch_bounds__(256, 2) void conv_generic_dma_kernel(ConvArgs a, Ge
 #pragma unroll
     for (int u = 0; u < GEN_NST - 1; u++)
         if (u < nsteps) issue(u, u);
+    gen_params<BN>(a, g, n0, prm);
     int rbuf = 0;                                      // ring slot of step s
     for (int st = 0; st < nsteps; st++) {
         if (st + GEN_NST - 2 < nsteps) dma_wait_barrier<(GEN_NST - 2) * LPS>();
@@ -388,11 +601,11 @@ __global__ __launch_bounds__(256, 2) void conv_generic_dma_kernel(ConvArgs a, Ge
             for (int i = 0; i < MI; i++)
 #pragma unroll
                 for (int j = 0; j < NJ; j++)
-                    acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[i], bf[j], acc[i][j], 0, 0, 0);
+                    acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(bf[j], af[i], acc[i][j], 0, 0, 0);
         }
         rbuf = rbuf == GEN_NST - 1 ? 0 : rbuf + 1;
     }
-    gen_epilogue<MI, NJ>(acc, a, g, m0, n0, wm * (BM / 2), wn * (BN / 2));
+    gen_epilogue<BM, BN, LUT>(acc, a, g, m0, n0, wm * (BM / 2), wn * (BN / 2), smem, prm);
 }
 
 // Tile shape of a launch: 128-wide in N above 64 output channels, 128-high
@@ -408,20 +621,26 @@ GenTile gen_tile(long long M, int cin, int cout) {
     return t;
 }
 
+template <int RUN, int BM, int BN, bool LUT>
+void launch_tile(dim3 gd, hipStream_t s, const ConvArgs& a, const GenGeom& g) {
+    if constexpr (RUN == 16) hipLaunchKernelGGL((conv_generic_dma_kernel<BM, BN, LUT>), gd, dim3(256), 0, s, a, g);
+    else hipLaunchKernelGGL((conv_generic_kernel<RUN, BM, BN, LUT>), gd, dim3(256), 0, s, a, g);
+}
+
+template <int RUN, bool LUT>
+void launch_run(GenTile t, dim3 gd, hipStream_t s, const ConvArgs& a, const GenGeom& g) {
+    if (t.bm == 128 && t.bn == 128) launch_tile<RUN, 128, 128, LUT>(gd, s, a, g);
+    else if (t.bm == 128) launch_tile<RUN, 128, 64, LUT>(gd, s, a, g);
+    else if (t.bn == 128) launch_tile<RUN, 64, 128, LUT>(gd, s, a, g);
+    else launch_tile<RUN, 64, 64, LUT>(gd, s, a, g);
+}
+
+// (kernels with the BN tables in LDS are separate: the tables of 128 channels
+// take 34 KB)
 template <int RUN>
 void launch_run(GenTile t, dim3 gd, hipStream_t s, const ConvArgs& a, const GenGeom& g) {
-    const dim3 bd(256);
-    if constexpr (RUN == 16) {
-        if (t.bm == 128 && t.bn == 128) hipLaunchKernelGGL((conv_generic_dma_kernel<128, 128>), gd, bd, 0, s, a, g);
-        else if (t.bm == 128) hipLaunchKernelGGL((conv_generic_dma_kernel<128, 64>), gd, bd, 0, s, a, g);
-        else if (t.bn == 128) hipLaunchKernelGGL((conv_generic_dma_kernel<64, 128>), gd, bd, 0, s, a, g);
-        else hipLaunchKernelGGL((conv_generic_dma_kernel<64, 64>), gd, bd, 0, s, a, g);
-    } else {
-        if (t.bm == 128 && t.bn == 128) hipLaunchKernelGGL((conv_generic_kernel<RUN, 128, 128>), gd, bd, 0, s, a, g);
-        else if (t.bm == 128) hipLaunchKernelGGL((conv_generic_kernel<RUN, 128, 64>), gd, bd, 0, s, a, g);
-        else if (t.bn == 128) hipLaunchKernelGGL((conv_generic_kernel<RUN, 64, 128>), gd, bd, 0, s, a, g);
-        else hipLaunchKernelGGL((conv_generic_kernel<RUN, 64, 64>), gd, bd, 0, s, a, g);
-    }
+    if ((a.flags & FFK_EPI_BN) && !a.out_i32) launch_run<RUN, true>(t, gd, s, a, g);
+    else launch_run<RUN, false>(t, gd, s, a, g);
 }
 
 }  // namespace
@@ -444,6 +663,9 @@ int ff_conv_generic_launch(const ConvArgs& a, const ffk_conv_desc* d, hipStream_
     // alignment in memory (a tensor base that is not 16-byte aligned takes
     // the byte gather)
     const int run = (d->cin == 3 || d->cin % 8 || ((uintptr_t)d->in & 15)) ? 0 : d->cin % 16 ? 8 : 16;
+    uintptr_t bits = (uintptr_t)d->cout | (uintptr_t)d->out | (uintptr_t)d->out_bn;
+    if (d->flags & FFK_EPI_ADD) bits |= (uintptr_t)d->add_src;
+    g.vec = bits & 3 ? 1 : bits & 4 ? 4 : bits & 8 ? 8 : 16;
     // The channel-run gathers address the int8 input with 32-bit offsets: a
     // batch whose input or output tensor reaches 2 GiB runs as several
     // launches over consecutive image ranges (images are independent).  The
