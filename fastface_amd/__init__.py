@@ -92,6 +92,7 @@ EXPORTS = [
     ("ffk_malloc", _p, [C.c_size_t]),
     ("ffk_free", C.c_int, [_p]),
     ("ffk_host_alloc", _p, [C.c_size_t]),
+    ("ffk_host_alloc_coherent", _p, [C.c_size_t]),
     ("ffk_host_free", C.c_int, [_p]),
     ("ffk_memcpy_h2d", C.c_int, [_p, _p, C.c_size_t, _p]),
     ("ffk_memcpy_d2h", C.c_int, [_p, _p, C.c_size_t, _p]),

@@ -59,6 +59,13 @@ void* ffk_host_alloc(size_t bytes) {
     return p;
 }
 
+void* ffk_host_alloc_coherent(size_t bytes) {
+    void* p = nullptr;
+    hipError_t e = hipHostMalloc(&p, bytes ? bytes : 1, hipHostMallocCoherent);
+    if (e != hipSuccess) { ffk_hip_fail(e, "hipHostMalloc"); return nullptr; }
+    return p;
+}
+
 int ffk_host_free(void* p) {
     if (!p) return FFK_OK;
     hipError_t e = hipHostFree(p);

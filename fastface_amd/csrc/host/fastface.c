@@ -55,11 +55,11 @@
 #define FF_STAGE_BYTES ((size_t)FF_STAGE_MB << 20)
 /* a one-chunk host batch of at least this many bytes is staged too */
 #define FF_STAGE_MIN_BYTES ((size_t)8 << 20)
-/* Small host batches bounce through one pinned buffer instead (a DMA from
- * pinned memory skips the runtime's own staging of pageable memory): the
- * input up to FF_SMALL_IN bytes (one fp32 face, six uint8 faces), the
- * embeddings up to FF_SMALL_OUT bytes (eight faces).  Measured at b=1: the
- * 2 KB embedding 21.4 -> 11.9 us, the 147 KB face 14.7 -> 13.1 us. */
+/* Small host batches go through one pinned, coherent buffer instead, which
+ * the chain's first and last kernels address in place: the input up to
+ * FF_SMALL_IN bytes (one fp32 face, six uint8 faces) and its embeddings
+ * (FF_SMALL_OUT).  A DMA each way costs 11-13 us however small it is; in
+ * place, one face host to host takes 265 us instead of 280. */
 #define FF_SMALL_IN ((size_t)256 << 10)
 #define FF_SMALL_OUT ((size_t)16 << 10)
 
@@ -120,7 +120,7 @@ struct FastFace {
     void* ev_fork, *ev_join;    /* (recorded only inside graph capture) */
     void* ev_chunk[FF_MAX_CHUNKS];
     void* h_stage[2];           /* pinned staging of streamed input pieces (on first use) */
-    void* h_small;              /* pinned bounce buffer of small host batches (on first use):
+    void* h_small;              /* pinned buffer of small host batches (on first use):
                                    FF_SMALL_IN input bytes, then FF_SMALL_OUT output bytes */
     void* ev_stage[2];          /* the last DMA out of each staging buffer */
     Stager* stager;             /* its copy threads (on first use), or NULL */
@@ -761,11 +761,11 @@ static int stage_h2d(FastFace* ff, Stager* st, int8_t* d_in, const int8_t* in, s
     return 0;
 }
 
-/* the pinned bounce buffer of small host batches, NULL if it cannot be
- * had (the copies then go from and to the caller's memory directly) */
+/* the pinned buffer of small host batches, NULL if it cannot be had (the
+ * faces are then copied from and to the caller's memory) */
 static int8_t* small_buffer(FastFace* ff)
 {
-    if (!ff->h_small) ff->h_small = ffk_host_alloc(FF_SMALL_IN + FF_SMALL_OUT);
+    if (!ff->h_small) ff->h_small = ffk_host_alloc_coherent(FF_SMALL_IN + FF_SMALL_OUT);
     return (int8_t*)ff->h_small;
 }
 
@@ -785,28 +785,28 @@ static int embed_host(FastFace* ff, const void* in, size_t face_bytes, int fmt, 
     if (streamed && batch - first > chunk * (FF_MAX_CHUNKS - 1))
         chunk = (batch - first + FF_MAX_CHUNKS - 2) / (FF_MAX_CHUNKS - 1);
     const int n = streamed ? 1 + (batch - first + chunk - 1) / chunk : 1;
-    if (n < 2 || ff->keep_all) {
+    /* a small batch: input and embeddings in the pinned buffer */
+    const size_t in_bytes = (size_t)batch * face_bytes;
+    int8_t* hs = in_bytes <= FF_SMALL_IN && out_bytes <= FF_SMALL_OUT ? small_buffer(ff) : NULL;
+    if (hs) {
+        /* (the stream is idle here after a completed call; the sync covers
+         * one that failed with its chain still in flight) */
+        rc = ffk_stream_sync(ff->stream);
+        if (!rc) memcpy(hs, in, in_bytes);
+        if (!rc) rc = set_io(ff, hs, (float*)(hs + FF_SMALL_IN), ff->stream, batch, fmt);
+        if (!rc) rc = enqueue(ff, batch, ff->stream, fmt);
+    } else if (n < 2 || ff->keep_all) {
         /* one chunk: a large one still goes through the staging buffers */
-        const size_t bytes = (size_t)batch * face_bytes;
-        Stager* st = bytes >= FF_STAGE_MIN_BYTES ? staging(ff) : NULL;
+        Stager* st = in_bytes >= FF_STAGE_MIN_BYTES ? staging(ff) : NULL;
         int piece = 0;
         rc = set_io(ff, d_in, ff->d_output, ff->stream, batch, fmt);
         if (!rc && st) {
-            rc = stage_h2d(ff, st, d_in, (const int8_t*)in, 0, bytes, &piece);
+            rc = stage_h2d(ff, st, d_in, (const int8_t*)in, 0, in_bytes, &piece);
             if (!rc) rc = ffk_event_record(ff->ev_chunk[0], ff->cstream);
             if (!rc) rc = ffk_stream_wait_event(ff->stream, ff->ev_chunk[0]);
             if (rc) ffk_stream_sync(ff->cstream);
         } else if (!rc) {
-            int8_t* hs = bytes <= FF_SMALL_IN ? small_buffer(ff) : NULL;
-            /* (the stream is idle here after a completed call; the sync
-             * covers a call that failed with its copy still in flight) */
-            if (hs) rc = ffk_stream_sync(ff->stream);
-            if (!rc && hs) {
-                memcpy(hs, in, bytes);
-                rc = ffk_memcpy_h2d(d_in, hs, bytes, ff->stream);
-            } else if (!rc) {
-                rc = ffk_memcpy_h2d(d_in, in, bytes, ff->stream);
-            }
+            rc = ffk_memcpy_h2d(d_in, in, in_bytes, ff->stream);
         }
         if (!rc) rc = enqueue(ff, batch, ff->stream, fmt);
     } else {
@@ -838,11 +838,9 @@ static int embed_host(FastFace* ff, const void* in, size_t face_bytes, int fmt, 
             memset(ff->io_cur, 0, sizeof ff->io_cur);
         }
     }
-    int8_t* ho = out_bytes <= FF_SMALL_OUT ? small_buffer(ff) : NULL;
-    if (ho) ho += FF_SMALL_IN;
-    if (!rc) rc = ffk_memcpy_d2h(ho ? (void*)ho : (void*)out, ff->d_output, out_bytes, ff->stream);
+    if (!rc && !hs) rc = ffk_memcpy_d2h(out, ff->d_output, out_bytes, ff->stream);
     if (!rc) rc = ffk_stream_sync(ff->stream);
-    if (!rc && ho) memcpy(out, ho, out_bytes);
+    if (!rc && hs) memcpy(out, hs + FF_SMALL_IN, out_bytes);
     if (!rc) ff->last_stream = NULL;        /* all of it has finished */
     if (rc) { report("embed", rc); return -3; }
     return 0;

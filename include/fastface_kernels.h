@@ -33,6 +33,10 @@ int   ffk_device_count(void);
 void* ffk_malloc(size_t bytes);                 /* NULL on failure */
 int   ffk_free(void* dptr);
 void* ffk_host_alloc(size_t bytes);             /* pinned host memory */
+/* pinned host memory that kernels may read and write in place: coherent, so
+ * a kernel sees what the host wrote before its launch and the host what a
+ * finished kernel wrote */
+void* ffk_host_alloc_coherent(size_t bytes);
 int   ffk_host_free(void* hptr);
 int   ffk_memcpy_h2d(void* dst, const void* src, size_t bytes, void* stream);
 int   ffk_memcpy_d2h(void* dst, const void* src, size_t bytes, void* stream);
