@@ -63,8 +63,8 @@
 #define FF_SMALL_IN ((size_t)256 << 10)
 #define FF_SMALL_OUT ((size_t)16 << 10)
 
-/* Batches of FF_SPLIT_MIN faces or more run as two halves, each on its own
- * stream inside the one captured graph (a fork and a join), both launched
+/* Batches of FF_SPLIT_MIN faces or more run as two halves, each its own
+ * captured graph on its own stream between a fork and a join, both launched
  * with FFK_SHARED_GPU (each layer takes the tiling the two halves' grids
  * together fill the GPU with).  A layer's kernel of one half fills the CUs
  * the other half's kernel leaves idle: the last, partly filled round of
@@ -81,7 +81,11 @@
 #define FF_SPLIT_MIN 24
 
 /* one captured chain per (batch, input format: 0 fp32 faces, 1 uint8 RGB) */
-typedef struct { int batch, fmt; void* exec; } GraphEntry;
+typedef struct {
+    int batch, fmt;
+    void* exec;                 /* the chain, or its first half */
+    void* exec2;                /* its second half, or NULL */
+} GraphEntry;
 
 /* Stream ordering.  A context's device state (the I/O descriptor, the
  * activation buffers, the split-K workspace and its counters, the captured
@@ -117,7 +121,7 @@ struct FastFace {
                                    [0..1] set_io, [2(1 + k)..] chunk k */
     void* cstream;              /* host-to-device copies of streamed chunks */
     void* sstream;              /* the second half of a split chain */
-    void* ev_fork, *ev_join;    /* (recorded only inside graph capture) */
+    void* ev_fork, *ev_join;    /* around the second half */
     void* ev_chunk[FF_MAX_CHUNKS];
     void* h_stage[2];           /* pinned staging of streamed input pieces (on first use) */
     void* h_small;              /* pinned buffer of small host batches (on first use):
@@ -166,7 +170,10 @@ static int mark_enqueued(FastFace* ff, void* stream)
 
 static void drop_graphs(FastFace* ff)
 {
-    for (int i = 0; i < ff->n_graphs; i++) ffk_graph_destroy(ff->graphs[i].exec);
+    for (int i = 0; i < ff->n_graphs; i++) {
+        ffk_graph_destroy(ff->graphs[i].exec);
+        ffk_graph_destroy(ff->graphs[i].exec2);
+    }
     ff->n_graphs = 0;
     ff->graph_rr = 0;
 }
@@ -435,64 +442,88 @@ static int run_direct(FastFace* ff, int batch, void* stream, int fmt)
     return run_part(ff, 0, 0, batch, stream, fmt, 0);
 }
 
-/* The chain as captured: one, or two halves forked onto the second stream
- * and joined back (the join is recorded even after an error, so that the
- * capture can end). */
-static int run_captured(FastFace* ff, int batch, int fmt)
+/* Half `part` of a `batch` chain (part 0 of an unsplit one: all of it)
+ * captured on the stream it is named after; 0 and *exec, or an error. */
+static int capture_part(FastFace* ff, int part, int batch, int fmt, void** exec)
 {
     const int na = split_at(ff, batch);
-    if (!na) return run_direct(ff, batch, ff->stream, fmt);
-    int rc = ffk_event_record(ff->ev_fork, ff->stream);
+    void* stream = part ? ff->sstream : ff->stream;
+    *exec = NULL;
+    int rc = ffk_graph_begin(stream);
     if (rc) return rc;
-    rc = ffk_stream_wait_event(ff->sstream, ff->ev_fork);
-    if (!rc) rc = run_part(ff, 0, 0, na, ff->stream, fmt, 1);
-    if (!rc) rc = run_part(ff, 1, (size_t)na * ff->plan.max_face_bytes, batch - na, ff->sstream, fmt, 1);
-    int rj = ffk_event_record(ff->ev_join, ff->sstream);
-    if (!rj) rj = ffk_stream_wait_event(ff->stream, ff->ev_join);
-    return rc ? rc : rj;
+    if (!na) rc = run_direct(ff, batch, stream, fmt);
+    else if (part == 0) rc = run_part(ff, 0, 0, na, stream, fmt, 1);
+    else rc = run_part(ff, 1, (size_t)na * ff->plan.max_face_bytes, batch - na, stream, fmt, 1);
+    const int re = ffk_graph_end(stream, exec);
+    if (rc && *exec) { ffk_graph_destroy(*exec); *exec = NULL; }
+    return rc ? rc : re;
 }
 
-/* The captured chain for (batch, fmt), capturing it on first use.  A full
- * cache evicts round-robin, never the entries holding `keep` or `keep2`
+/* The captured chain for (batch, fmt), capturing it on first use, or NULL.
+ * A full cache evicts round-robin, never the entries `keep` or `keep2`
  * (chains the caller is about to launch); an evicted chain may still be in
  * flight, so the context's work is waited for before it is destroyed. */
-static void* graph_for(FastFace* ff, int batch, int fmt, const void* keep, const void* keep2)
+static const GraphEntry* graph_for(FastFace* ff, int batch, int fmt, const GraphEntry* keep, const GraphEntry* keep2)
 {
     for (int i = 0; i < ff->n_graphs; i++)
-        if (ff->graphs[i].batch == batch && ff->graphs[i].fmt == fmt) return ff->graphs[i].exec;
-    if (ffk_graph_begin(ff->stream)) return NULL;
-    int rc = run_captured(ff, batch, fmt);
-    void* exec = NULL;
-    int rc2 = ffk_graph_end(ff->stream, &exec);
-    if (rc || rc2) { if (exec) ffk_graph_destroy(exec); return NULL; }
+        if (ff->graphs[i].batch == batch && ff->graphs[i].fmt == fmt) return &ff->graphs[i];
+    GraphEntry e = {batch, fmt, NULL, NULL};
+    if (capture_part(ff, 0, batch, fmt, &e.exec)) return NULL;
+    if (split_at(ff, batch) && capture_part(ff, 1, batch, fmt, &e.exec2)) {
+        ffk_graph_destroy(e.exec);
+        return NULL;
+    }
     int slot;
     if (ff->n_graphs < FF_MAX_GRAPHS) {
         slot = ff->n_graphs++;
     } else {
         slot = ff->graph_rr;
-        while (ff->graphs[slot].exec == keep || ff->graphs[slot].exec == keep2) slot = (slot + 1) % FF_MAX_GRAPHS;
+        while (&ff->graphs[slot] == keep || &ff->graphs[slot] == keep2) slot = (slot + 1) % FF_MAX_GRAPHS;
         ff->graph_rr = (slot + 1) % FF_MAX_GRAPHS;
-        if (drain(ff) || ffk_stream_sync(ff->stream)) { ffk_graph_destroy(exec); return NULL; }
+        if (drain(ff) || ffk_stream_sync(ff->stream)) {
+            ffk_graph_destroy(e.exec);
+            ffk_graph_destroy(e.exec2);
+            return NULL;
+        }
         ffk_graph_destroy(ff->graphs[slot].exec);
+        ffk_graph_destroy(ff->graphs[slot].exec2);
     }
-    ff->graphs[slot].batch = batch;
-    ff->graphs[slot].fmt = fmt;
-    ff->graphs[slot].exec = exec;
-    return exec;
+    ff->graphs[slot] = e;
+    return &ff->graphs[slot];
+}
+
+/* A captured chain on `stream`; two halves fork onto the second stream and
+ * join back.  As two one-stream graphs a launch costs the host about 15 us;
+ * as one graph of two branches the runtime enqueued its 108 kernels one by
+ * one, 80-120 us more for a batch on an idle GPU (24 faces 695 -> 597 us, 203
+ * faces 1819 -> 1617, calls with other buffers each time).  (The join is
+ * made even after an error, so that nothing is left behind on the second
+ * stream.) */
+static int launch_chain(FastFace* ff, const GraphEntry* g, void* stream)
+{
+    if (!g->exec2) return ffk_graph_launch(g->exec, stream);
+    int rc = ffk_event_record(ff->ev_fork, stream);
+    if (!rc) rc = ffk_stream_wait_event(ff->sstream, ff->ev_fork);
+    if (rc) return rc;
+    rc = ffk_graph_launch(g->exec, stream);
+    if (!rc) rc = ffk_graph_launch(g->exec2, ff->sstream);
+    int rj = ffk_event_record(ff->ev_join, ff->sstream);
+    if (!rj) rj = ffk_stream_wait_event(stream, ff->ev_join);
+    return rc ? rc : rj;
 }
 
 /* Enqueue one batch whose I/O pointers are already in d_io: ordered after
  * the context's last enqueue (whatever stream that was on), then marked as
- * the new last one.  `exec`: a chain already looked up, or NULL. */
-static int enqueue_exec(FastFace* ff, int batch, void* stream, int fmt, void* exec)
+ * the new last one.  `g`: a chain already looked up, or NULL. */
+static int enqueue_chain(FastFace* ff, int batch, void* stream, int fmt, const GraphEntry* g)
 {
     int rc = order_after_last(ff, stream);
     if (rc) return rc;
     if (ff->keep_all) {
         rc = run_direct(ff, batch, stream, fmt);
     } else {
-        void* g = exec ? exec : graph_for(ff, batch, fmt, NULL, NULL);
-        rc = g ? ffk_graph_launch(g, stream) : FFK_ERR_HIP;
+        if (!g) g = graph_for(ff, batch, fmt, NULL, NULL);
+        rc = g ? launch_chain(ff, g, stream) : FFK_ERR_HIP;
     }
     if (!rc) rc = mark_enqueued(ff, stream);
     return rc;
@@ -500,7 +531,7 @@ static int enqueue_exec(FastFace* ff, int batch, void* stream, int fmt, void* ex
 
 static int enqueue(FastFace* ff, int batch, void* stream, int fmt)
 {
-    return enqueue_exec(ff, batch, stream, fmt, NULL);
+    return enqueue_chain(ff, batch, stream, fmt, NULL);
 }
 
 FastFace* fastface_create(const char* ffw4_path)
@@ -814,9 +845,9 @@ static int embed_host(FastFace* ff, const void* in, size_t face_bytes, int fmt, 
          * lookup may not evict the chains looked up before it), and launch
          * them directly */
         const int last = batch - first - (n - 2) * chunk;
-        void* g_first = graph_for(ff, first, fmt, NULL, NULL);
-        void* g_chunk = g_first && n > 2 ? graph_for(ff, chunk, fmt, g_first, NULL) : g_first;
-        void* g_last = g_chunk ? graph_for(ff, last, fmt, g_first, g_chunk) : NULL;
+        const GraphEntry* g_first = graph_for(ff, first, fmt, NULL, NULL);
+        const GraphEntry* g_chunk = g_first && n > 2 ? graph_for(ff, chunk, fmt, g_first, NULL) : g_first;
+        const GraphEntry* g_last = g_chunk ? graph_for(ff, last, fmt, g_first, g_chunk) : NULL;
         if (!g_first || !g_chunk || !g_last) rc = FFK_ERR_HIP;
         Stager* st = rc ? NULL : staging(ff);
         int piece = 0;
@@ -829,7 +860,7 @@ static int embed_host(FastFace* ff, const void* in, size_t face_bytes, int fmt, 
             ffk_io* slot = &ff->h_io[2 * (1 + k)];
             io_pair(ff, slot, d_in + b0 * face_bytes, ff->d_output + b0 * FASTFACE_OUTPUT_N, nb, fmt);
             if (!rc) rc = ffk_memcpy_h2d(ff->d_io, slot, 2 * sizeof(ffk_io), ff->stream);
-            if (!rc) rc = enqueue_exec(ff, nb, ff->stream, fmt, k == 0 ? g_first : (k + 1 < n ? g_chunk : g_last));
+            if (!rc) rc = enqueue_chain(ff, nb, ff->stream, fmt, k == 0 ? g_first : (k + 1 < n ? g_chunk : g_last));
             if (!rc) memcpy(ff->io_cur, slot, sizeof ff->io_cur);
         }
         if (rc) {           /* leave no copy or chunk running into the buffers */
