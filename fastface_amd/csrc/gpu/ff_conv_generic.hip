@@ -25,6 +25,9 @@ struct GenGeom {
     int cin, cout, kh, kw, stride, pad, hin, win, hout, wout;
     int ktot;       // kh * kw * cin
     int kpad;       // ktot rounded up to whole 64-byte weight steps
+    int d_ci, d_tw, d_th;    // 64 = d_ci + cin * (d_tw + kw * d_th): one K step in (channel, tap column, tap row)
+    int row_skip;        // (win - kw) * cin: elements a tap-row step skips
+    unsigned mag_hw, mag_wo; // multipliers of the divisions by hout*wout (below 128) and wout, 0: divide
     unsigned in_bytes;   // the launch's int8 input tensor (below 2 GiB)
     int vec;             // bytes per access of the int8 outputs and the residual
 };
@@ -45,6 +48,42 @@ __device__ __forceinline__ KCursor kcursor_at(const GenGeom& g, int k) {
     c.tw = tap - c.th * g.kw;
     c.off = (c.th * g.win + c.tw) * g.cin + c.ci;
     return c;
+}
+
+// The cursor one 64-element K step on, without branches: each digit of the
+// mixed-radix position wraps at most once.  (The K loop's address arithmetic is
+// what its waves issue between MFMAs: with a loop over the wraps, 64-bit row
+// divisions before it and four-way bounds checks, 3x3 256->256 @20 at 64 faces
+// took 28.7 us, now 24.6; 5x5 63.4, now 55-57.)
+__device__ __forceinline__ void kcursor_next(KCursor& c, const GenGeom& g) {
+    c.k += 64;
+    c.ci += g.d_ci;
+    const bool w0 = c.ci >= g.cin;
+    c.ci -= w0 ? g.cin : 0;
+    c.tw += g.d_tw + w0;
+    const bool w1 = c.tw >= g.kw;
+    c.tw -= w1 ? g.kw : 0;
+    const int dth = g.d_th + w1;
+    c.th += dth;
+    c.off += 64 + dth * g.row_skip;
+}
+
+// Image and in-image position of the tile's pixel m0 + r: b0, rem0 those of
+// the tile's first pixel (uniform), r < 128.
+__device__ __forceinline__ void gen_pixel(const GenGeom& g, int hw, int b0, int rem0, int r, int& b, int& oh, int& ow) {
+    unsigned rem = (unsigned)(rem0 + r);
+    b = b0;
+    if (hw >= 128) {                                  // at most one image further
+        const bool w = rem >= (unsigned)hw;
+        rem -= w ? hw : 0;
+        b += w;
+    } else {
+        const unsigned q = g.mag_hw ? __umulhi(rem, g.mag_hw) : rem;       // (hw 1: rem images on)
+        b += (int)q;
+        rem -= q * hw;
+    }
+    oh = (int)(g.mag_wo ? __umulhi(rem, g.mag_wo) : rem / (unsigned)g.wout);
+    ow = (int)rem - oh * g.wout;
 }
 
 // Moves the cursor n elements on without a division: each channel wrap is
@@ -124,8 +163,8 @@ __device__ __forceinline__ v4i gather_a(const ConvArgs& a, const GenGeom& g, __a
 // staging tile, which then leaves as 16-byte chunks of a pixel's channels.
 // (Stored straight from registers a 128x128 tile was 64 byte stores per lane
 // of 32 bytes a row, and the BN output a table gather per element: 3x3 96->96
-// @45 PReLU at 33 faces 27.4 us, now 20.1; 96->128 @35 residual+BN at 196 faces
-// 129 us, now 64.)
+// @45 PReLU at 33 faces 27.4 us, now 17.0; 96->128 @35 residual+BN at 196 faces
+// 129 us, now 60.)
 
 // Channels per vector of the int8 tensors' accesses: 16, 8, 4 or 1 bytes, the
 // largest that divides the channel count and every base address.
@@ -219,9 +258,22 @@ __device__ __forceinline__ void gen_lut_store(const v4i (&t)[4], int8_t* lut) {
     }
 }
 
+// Four int32 saturated to int8, packed (v_ashr_pk_i8_i32 saturates two).  An
+// in-range requant value truncated to int32 and then saturated is the value
+// the fp32 clamp before the truncation gives: the bounds are integers.
+__device__ __forceinline__ uint32_t pack_sat_i8(int a, int b, int c, int d) {
+    const uint32_t lo = (uint16_t)__builtin_amdgcn_ashr_pk_i8_i32((unsigned)a, (unsigned)b, 0);
+    const uint32_t hi = (uint16_t)__builtin_amdgcn_ashr_pk_i8_i32((unsigned)c, (unsigned)d, 0);
+    return __builtin_amdgcn_perm(hi, lo, 0x05040100u);
+}
+
 // The wave's MI x NJ blocks at tile (m0 + wr, n0 + wc) to the staging tile
-// `stage` and X to memory.  prm: the tile's parameter rows.
-template <int MI, int NJ, int BN, bool RNG>
+// `stage` and X to memory.  prm: the tile's parameter rows.  RANGE and PRELU
+// as in wave_epi_i8 (0 / 1 with the flags read at run time: the general
+// form).  PIPE: a group's
+// parameters are read one group ahead of its arithmetic (not beside the BN
+// tables in flight: 128 registers keep four workgroups per CU).
+template <int MI, int NJ, int BN, int RANGE, int PRELU, bool PIPE>
 __device__ __forceinline__ void gen_epi_i8(const v16i (&acc)[MI][NJ], const ConvArgs& a, const GenGeom& g, long long m0,
                                            int n0, int wc, int8_t* stage, const float* prm) {
     typedef float v4f __attribute__((ext_vector_type(4)));
@@ -229,73 +281,94 @@ __device__ __forceinline__ void gen_epi_i8(const v16i (&acc)[MI][NJ], const Conv
     constexpr int CH = NJ * 2, RPI = 64 / CH;          // 16-byte chunks per row, rows per chunk access
     const int lane = threadIdx.x & 63;
     const int lc = lane & 31, lh = lane >> 5;
-    const bool add = (a.flags & FFK_EPI_ADD) != 0, prelu = (a.flags & FFK_EPI_PRELU) != 0;
-    const bool insc = !RNG && (a.flags & FFK_EPI_INSCALE);
+    const bool add = RANGE != 2 && (a.flags & FFK_EPI_ADD), prelu = PRELU && (a.flags & FFK_EPI_PRELU);
+    const bool insc = RANGE == 0 && (a.flags & FFK_EPI_INSCALE);
     if (add) {
+        v4i v[MI * 32 / RPI];
+        auto fetch = [&](int vec) {
 #pragma unroll
-        for (int k = 0; k < MI * 32 / RPI; k++) {
-            const int row = lane / CH + k * RPI, n = n0 + wc + (lane % CH) * 16;
-            const long long m = m0 + row;
-            v4i v = {0, 0, 0, 0};
-            if (m < a.M && n < g.cout) v = chunk_load(a.add_src + (size_t)m * g.cout + n, g.cout - n, g.vec);
-            *reinterpret_cast<v4i*>(stage + row * P + (lane % CH) * 16) = v;
-        }
+            for (int k = 0; k < MI * 32 / RPI; k++) {
+                const int n = n0 + wc + (lane % CH) * 16;
+                const long long m = m0 + lane / CH + k * RPI;
+                v[k] = v4i{0, 0, 0, 0};
+                if (m < a.M && n < g.cout) v[k] = chunk_load(a.add_src + (size_t)m * g.cout + n, g.cout - n, vec);
+            }
+        };
+        if (g.vec == 16) fetch(16);
+        else fetch(g.vec);
+#pragma unroll
+        for (int k = 0; k < MI * 32 / RPI; k++)
+            *reinterpret_cast<v4i*>(stage + (lane / CH + k * RPI) * P + (lane % CH) * 16) = v[k];
         __builtin_amdgcn_wave_barrier();               // (the wave's own tile: its LDS accesses run in order)
     }
+    struct Prm { v4f ws, bias, inv, slope, adds; };
+    auto params = [&](int t) {                         // of group t: channels (t/4)*32 + (t%4)*8 + lh*4 ..
+        const float* pr = prm + wc + (t >> 2) * 32 + (t & 3) * 8 + lh * 4;
+        Prm p;
+        p.ws = *reinterpret_cast<const v4f*>(pr);
+        p.bias = *reinterpret_cast<const v4f*>(pr + BN);
+        p.inv = *reinterpret_cast<const v4f*>(pr + 4 * BN);
+        if (prelu) p.slope = *reinterpret_cast<const v4f*>(pr + 2 * BN);
+        if (add) p.adds = *reinterpret_cast<const v4f*>(pr + 3 * BN);
+        return p;
+    };
+    Prm nxt = params(0);
 #pragma unroll
-    for (int j = 0; j < NJ; j++)
+    for (int t = 0; t < NJ * 4; t++) {
+        const int j = t >> 2, q = t & 3;
+        const Prm p = nxt;
+        if (PIPE && t + 1 < NJ * 4) nxt = params(t + 1);
 #pragma unroll
-        for (int q = 0; q < 4; q++) {
-            const int c = j * 32 + q * 8 + lh * 4;     // first channel of the group in the wave's block
-            const float* pr = prm + wc + c;
-            const v4f ws = *reinterpret_cast<const v4f*>(pr), bias = *reinterpret_cast<const v4f*>(pr + BN);
-            const v4f inv = *reinterpret_cast<const v4f*>(pr + 4 * BN);
-            v4f slope = {0, 0, 0, 0}, adds = {0, 0, 0, 0};
-            if (prelu) slope = *reinterpret_cast<const v4f*>(pr + 2 * BN);
-            if (add) adds = *reinterpret_cast<const v4f*>(pr + 3 * BN);
+        for (int i = 0; i < MI; i++) {
+            uint32_t* d = reinterpret_cast<uint32_t*>(stage + (i * 32 + lc) * P + j * 32 + q * 8 + lh * 4);
+            const uint32_t res = add ? *d : 0u;
+            int v[4];
 #pragma unroll
-            for (int i = 0; i < MI; i++) {
-                uint32_t* t = reinterpret_cast<uint32_t*>(stage + (i * 32 + lc) * P + c);
-                const uint32_t res = add ? *t : 0u;
-                int v[4];
-#pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    float f = (float)acc[i][j][q * 4 + e];
-                    if (insc) f = f * a.in_scale;
-                    f = f * ws[e];
-                    f = f + bias[e];
-                    if (add) f = ff::add_residual(f, (int32_t)(int8_t)(res >> (8 * e)), adds[e]);
-                    if (prelu) f = ff::prelu(f, slope[e]);
-                    v[e] = RNG ? ff::requant_haz_in_range(f * inv[e]) : ff::requant_haz(f * inv[e]);
+            for (int e = 0; e < 4; e++) {
+                float f = (float)acc[i][j][q * 4 + e];
+                if (insc) f = f * a.in_scale;
+                f = f * p.ws[e];
+                f = f + p.bias[e];
+                if (add) f = ff::add_residual(f, (int32_t)(int8_t)(res >> (8 * e)), p.adds[e]);
+                if (PRELU == 1 && prelu) f = ff::prelu(f, p.slope[e]);
+                if (PRELU == 2 && prelu) f = ff::prelu_le1(f, p.slope[e]);
+                if (RANGE == 0) {
+                    v[e] = ff::requant_haz(f * p.inv[e]);
+                } else {                               // (truncated here, clamped by the pack)
+                    const float h = RANGE == 2 ? __builtin_fmaf(f, p.inv[e], copysignf(0.5f, f))
+                                               : f * p.inv[e] + copysignf(0.5f, f * p.inv[e]);
+                    v[e] = (int)h;
                 }
-                const uint32_t lo = __builtin_amdgcn_perm((uint32_t)v[1], (uint32_t)v[0], 0x0c0c0400u);
-                const uint32_t hi = __builtin_amdgcn_perm((uint32_t)v[3], (uint32_t)v[2], 0x0c0c0400u);
-                *t = __builtin_amdgcn_perm(hi, lo, 0x05040100u);
             }
-            asm volatile("" ::: "memory");             // one group at a time: bounds the live parameters
+            *d = pack_sat_i8(v[0], v[1], v[2], v[3]);
         }
+        asm volatile("" ::: "memory");                 // one group at a time: bounds the live parameters
+        if (!PIPE && t + 1 < NJ * 4) nxt = params(t + 1);
+    }
     __builtin_amdgcn_wave_barrier();
     const bool x_even = (a.flags & FFK_OUT_X_EVEN) != 0;
     if (!a.out) return;
+    auto flush = [&](int vec) {
 #pragma unroll
-    for (int k = 0; k < MI * 32 / RPI; k++) {
-        const int row = lane / CH + k * RPI, ch = (lane % CH) * 16, n = n0 + wc + ch;
-        const long long m = m0 + row;
-        if (m >= a.M || n >= g.cout) continue;
-        const v4i v = *reinterpret_cast<const v4i*>(stage + row * P + ch);
-        const size_t o = (size_t)m * g.cout + n;
-        if (!x_even) {
-            chunk_store(a.out + o, v, g.cout - n, g.vec);
-        } else {
-            const int hw = g.hout * g.wout;
-            const int bb = (int)(m / hw);
-            const int rem = (int)(m - (long long)bb * hw);
-            const int oh = rem / g.wout, ow = rem - oh * g.wout;
-            if (!((oh | ow) & 1))
-                chunk_store(a.out + (((size_t)bb * (g.hout / 2) + (oh >> 1)) * (g.wout / 2) + (ow >> 1)) * g.cout + n, v,
-                            g.cout - n, g.vec);
+        for (int k = 0; k < MI * 32 / RPI; k++) {
+            const int row = lane / CH + k * RPI, ch = (lane % CH) * 16, n = n0 + wc + ch;
+            const long long m = m0 + row;
+            if (m >= a.M || n >= g.cout) continue;
+            const v4i v = *reinterpret_cast<const v4i*>(stage + row * P + ch);
+            long long px = m;
+            if (x_even) {
+                const int hw = g.hout * g.wout;
+                const int bb = (int)(m / hw);
+                const int rem = (int)(m - (long long)bb * hw);
+                const int oh = rem / g.wout, ow = rem - oh * g.wout;
+                if ((oh | ow) & 1) continue;
+                px = ((long long)bb * (g.hout / 2) + (oh >> 1)) * (g.wout / 2) + (ow >> 1);
+            }
+            chunk_store(a.out + (size_t)px * g.cout + n, v, g.cout - n, vec);
         }
-    }
+    };
+    if (g.vec == 16) flush(16);
+    else flush(g.vec);
 }
 
 // BN(X) of the staging tile's j-th 32-channel block, through the round's
@@ -305,6 +378,7 @@ __device__ __forceinline__ void gen_bn_round(const ConvArgs& a, const GenGeom& g
                                              const int8_t* stage, const int8_t* lut) {
     const int lane = threadIdx.x & 63;
     const int ch = (lane & 1) * 16, n = n0 + j * 32 + ch;
+    auto flush = [&](int vec) {
 #pragma unroll
     for (int i = 0; i < MI; i++) {
         const int row = i * 32 + (lane >> 1);
@@ -323,8 +397,11 @@ __device__ __forceinline__ void gen_bn_round(const ConvArgs& a, const GenGeom& g
             const uint32_t hi = __builtin_amdgcn_perm(b[3], b[2], 0x0c0c0400u);
             w[d] = (int)__builtin_amdgcn_perm(hi, lo, 0x05040100u);
         }
-        chunk_store(a.out_bn + (size_t)m * g.cout + n, w, g.cout - n, g.vec);
+        chunk_store(a.out_bn + (size_t)m * g.cout + n, w, g.cout - n, vec);
     }
+    };
+    if (g.vec == 16) flush(16);
+    else flush(g.vec);
 }
 
 // All of it after the K loop: smem is the workgroup's LDS (the operands are
@@ -366,10 +443,17 @@ __device__ __forceinline__ void gen_epilogue(const v16i (&acc)[BM / 64][BN / 64]
     v4i t[4];
     if constexpr (LUT) gen_lut_load<NJ>(a, g, n0, 0, t);
     __syncthreads();                                   // every wave is done with the operands
-    if ((a.flags & FFK_EPI_IN_RANGE) && !(a.flags & FFK_EPI_INSCALE))
-        gen_epi_i8<MI, NJ, BN, true>(acc, a, g, m0 + wr, n0, wc, stage, prm);
-    else
-        gen_epi_i8<MI, NJ, BN, false>(acc, a, g, m0 + wr, n0, wc, stage, prm);
+    const int f = a.flags;
+    const bool pr = (f & FFK_EPI_PRELU) != 0;
+    const bool rng = (f & FFK_EPI_IN_RANGE) && !(f & FFK_EPI_INSCALE) && (!pr || (f & FFK_EPI_PRELU_LE1));
+    const bool fma = rng && (f & FFK_EPI_FMA_TAIL) && !(f & FFK_EPI_ADD);
+#define FF_GEN_EPI(RG, PR) gen_epi_i8<MI, NJ, BN, RG, PR, !LUT>(acc, a, g, m0 + wr, n0, wc, stage, prm)
+    if (!rng) FF_GEN_EPI(0, 1);
+    else if (fma && pr) FF_GEN_EPI(2, 2);
+    else if (fma) FF_GEN_EPI(2, 0);
+    else if (pr) FF_GEN_EPI(1, 2);
+    else FF_GEN_EPI(1, 0);
+#undef FF_GEN_EPI
     if constexpr (LUT) {
 #pragma unroll
         for (int j = 0; j < NJ; j++) {
@@ -391,7 +475,7 @@ __device__ __forceinline__ void gen_epilogue(const v16i (&acc)[BM / 64][BN / 64]
 // operand per MAC: every staged A row serves BN output channels, every B row
 // BM output pixels.
 template <int RUN, int BM, int BN, bool LUT>
-__global__ __launch_bounds__(256) void conv_generic_kernel(ConvArgs a, GenGeom g) {
+__global__ __launch_bounds__(256, 3) void conv_generic_kernel(ConvArgs a, GenGeom g) {
     constexpr int AR = BM / 64, BR = BN / 64;          // operand rows each thread stages
     constexpr int MI = BM / 64, NJ = BN / 64;          // 32x32 blocks per wave (2 x 2 waves)
     // one 64-byte K step per barrier pair (two or four steps' pieces staged
@@ -419,19 +503,15 @@ __global__ __launch_bounds__(256) void conv_generic_kernel(ConvArgs a, GenGeom g
     bool mrow[AR];
     int ih0[AR], iw0[AR];
     long long base[AR];          // element offset of the row's tap (0, 0) input pixel
+    const int b0 = (int)((unsigned)m0 / (unsigned)hw), rem0 = (int)((unsigned)m0 - (unsigned)b0 * hw);
 #pragma unroll
     for (int i = 0; i < AR; i++) {
-        const long long m = m0 + r + 64 * i;
-        mrow[i] = m < a.M;
-        ih0[i] = 0; iw0[i] = 0; base[i] = 0;
-        if (mrow[i]) {
-            const int b = (int)(m / hw);
-            const int rem = (int)(m - (long long)b * hw);
-            const int oh = rem / g.wout;
-            ih0[i] = oh * g.stride - g.pad;
-            iw0[i] = (rem - oh * g.wout) * g.stride - g.pad;
-            base[i] = (((long long)b * g.hin + ih0[i]) * g.win + iw0[i]) * g.cin;
-        }
+        mrow[i] = m0 + r + 64 * i < a.M;
+        int b, oh, ow;
+        gen_pixel(g, hw, b0, rem0, r + 64 * i, b, oh, ow);
+        ih0[i] = oh * g.stride - g.pad;
+        iw0[i] = ow * g.stride - g.pad;
+        base[i] = (((long long)b * g.hin + ih0[i]) * g.win + iw0[i]) * g.cin;
     }
     KCursor cur = kcursor_at(g, kq);
     const __amdgpu_buffer_rsrc_t r_in = ff_rsrc(a.in, RUN ? g.in_bytes : 0u);
@@ -464,7 +544,7 @@ __global__ __launch_bounds__(256) void conv_generic_kernel(ConvArgs a, GenGeom g
         for (int i = 0; i < BR; i++) *reinterpret_cast<v4i*>(Bs + (r + 64 * i) * PITCH + kq) = rb[i];
         __syncthreads();
         if (k0 + 64 < g.kpad) {
-            kcursor_step(cur, g, 64);
+            kcursor_next(cur, g);
 #pragma unroll
             for (int i = 0; i < AR; i++) ra[i] = gather_a<RUN>(a, g, r_in, x, mrow[i], base[i], ih0[i], iw0[i], cur);
 #pragma unroll
@@ -504,7 +584,7 @@ __global__ __launch_bounds__(256) void conv_generic_kernel(ConvArgs a, GenGeom g
 constexpr int GEN_NST = 2;
 
 template <int BM, int BN, bool LUT>
-__global__ __launch_bounds__(256, 2) void conv_generic_dma_kernel(ConvArgs a, GenGeom g) {
+__global__ __launch_bounds__(256, 4) void conv_generic_dma_kernel(ConvArgs a, GenGeom g) {
     constexpr int MI = BM / 64, NJ = BN / 64;          // 32x32 blocks per wave (2 x 2 waves)
     constexpr int A_BYTES = BM * 64, B_BYTES = BN * 64, STAGE = A_BYTES + B_BYTES;
     constexpr int A_LD = A_BYTES / (256 * 16), B_LD = B_BYTES / (256 * 16);
@@ -532,20 +612,16 @@ __global__ __launch_bounds__(256, 2) void conv_generic_dma_kernel(ConvArgs a, Ge
     const int sl = (lane & 15) ^ ((lane >> 4) & 3);
     const int p = sl & 3;
     int a_base[A_LD], a_ih0[A_LD], a_iw0[A_LD];
+    const int b0 = (int)((unsigned)m0 / (unsigned)hw), rem0 = (int)((unsigned)m0 - (unsigned)b0 * hw);
 #pragma unroll
     for (int j = 0; j < A_LD; j++) {
         const int r = ((j * 4 + wave) * 4 + (lane >> 4)) * 4 + (sl >> 2);
-        const long long m = m0 + r;
-        a_base[j] = 0; a_iw0[j] = 0;
-        a_ih0[j] = -(1 << 28);                         // a row past the batch fails every bounds check
-        if (m < a.M) {
-            const int b = (int)(m / hw);
-            const int rem = (int)(m - (long long)b * hw);
-            const int oh = rem / g.wout;
-            a_ih0[j] = oh * g.stride - g.pad;
-            a_iw0[j] = (rem - oh * g.wout) * g.stride - g.pad;
-            a_base[j] = ((b * g.hin + a_ih0[j]) * g.win + a_iw0[j]) * g.cin;
-        }
+        int b, oh, ow;
+        gen_pixel(g, hw, b0, rem0, r, b, oh, ow);
+        const int ih = oh * g.stride - g.pad;
+        a_iw0[j] = ow * g.stride - g.pad;
+        a_base[j] = ((b * g.hin + ih) * g.win + a_iw0[j]) * g.cin;
+        a_ih0[j] = m0 + r < a.M ? ih : -(1 << 28);     // a row past the batch fails every bounds check
     }
     unsigned b_off[B_LD];
 #pragma unroll
@@ -559,15 +635,15 @@ __global__ __launch_bounds__(256, 2) void conv_generic_dma_kernel(ConvArgs a, Ge
         const bool kin = cur.k < g.ktot;
 #pragma unroll
         for (int j = 0; j < A_LD; j++) {
-            const int ih = a_ih0[j] + cur.th, iw = a_iw0[j] + cur.tw;
-            const bool v = kin && ih >= 0 && ih < g.hin && iw >= 0 && iw < g.win;
+            const bool v = kin && (unsigned)(a_ih0[j] + cur.th) < (unsigned)g.hin &&
+                           (unsigned)(a_iw0[j] + cur.tw) < (unsigned)g.win;
             bdma16(r_in, v ? (unsigned)(a_base[j] + cur.off) : FF_OOB, 0u, sb + (j * 4 + wave) * 1024);
         }
         const unsigned wst = (unsigned)(st * g.cout * 64);
 #pragma unroll
         for (int j = 0; j < B_LD; j++)
-            bdma16(r_w, b_off[j] == FF_OOB ? FF_OOB : b_off[j] + wst, 0u, sb + A_BYTES + (j * 4 + wave) * 1024);
-        kcursor_step(cur, g, 64);
+            bdma16(r_w, b_off[j], wst, sb + A_BYTES + (j * 4 + wave) * 1024);
+        kcursor_next(cur, g);
     };
 
     const int wm = wave >> 1, wn = wave & 1;
@@ -659,6 +735,16 @@ int ff_conv_generic_launch(const ConvArgs& a, const ffk_conv_desc* d, hipStream_
     g.wout = (d->win + 2 * d->pad - d->kw) / d->stride + 1;
     g.ktot = d->kh * d->kw * d->cin;
     g.kpad = (g.ktot + FF_KSTEP - 1) / FF_KSTEP * FF_KSTEP;
+    g.d_ci = FF_KSTEP % g.cin;
+    g.d_tw = FF_KSTEP / g.cin % g.kw;
+    g.d_th = FF_KSTEP / g.cin / g.kw;
+    g.row_skip = (g.win - g.kw) * g.cin;
+    // multiplication by ceil(2^32 / d) divides m exactly while m * d < 2^32;
+    // m is below 128 + 128 for the first, below hout*wout for the second
+    auto mag = [](long long d) { return d < 2 ? 0u : (unsigned)((0x100000000ll + d - 1) / d); };
+    const long long px = (long long)g.hout * g.wout;
+    g.mag_hw = px < 128 ? mag(px) : 0u;
+    g.mag_wo = px * g.wout < 0x100000000ll ? mag(g.wout) : 0u;
     // channel runs are read as 8- / 16-byte vectors: they need the run's
     // alignment in memory (a tensor base that is not 16-byte aligned takes
     // the byte gather)
