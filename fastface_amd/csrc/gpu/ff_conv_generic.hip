@@ -16,6 +16,7 @@
 // from L2 / HBM for every output pixel.
 #include "ff_conv_table.h"
 #include "ff_numerics.h"
+#include "ff_wavek.h"
 
 #include <algorithm>
 
@@ -697,6 +698,16 @@ GenTile gen_tile(long long M, int cin, int cout) {
     return t;
 }
 
+// Grids of 64-row tiles up to one workgroup per CU and reductions of this many
+// 64-byte steps run on the wave-split kernel's tiles (ff_conv_wavek.hip): eight
+// waves instead of four, each with its own K steps and no barrier between them.
+// (us, four-wave tiles -> these: 5x5 s2 160->192 @7 residual+BN at 20 faces, 63
+// steps on 10 workgroups, 30.4 -> 14.6; 3x3 s2 160->384 @10 at 3 faces, 23
+// steps, 13.0 -> 8.2; 3x3 96->96 @45 at 8 faces, 14 steps on 254 workgroups,
+// 10.0 -> 7.8.  A four-stage ring in the four-wave tiles: 27.1, 12.6, 10.2,
+// and slower at 400 workgroups.)
+constexpr int GEN_WK_MIN_STEPS = 12;
+
 template <int RUN, int BM, int BN, bool LUT>
 void launch_tile(dim3 gd, hipStream_t s, const ConvArgs& a, const GenGeom& g) {
     if constexpr (RUN == 16) hipLaunchKernelGGL((conv_generic_dma_kernel<BM, BN, LUT>), gd, dim3(256), 0, s, a, g);
@@ -783,6 +794,14 @@ int ff_conv_generic_launch(const ConvArgs& a, const ffk_conv_desc* d, hipStream_
         }
         const GenTile t = gen_tile(as.M, d->cin, d->cout);
         const dim3 gd((unsigned)grid);
+        // (its vectors hold four channels; its pixel arithmetic needs M * hout*wout below 2^32, its
+        // K arithmetic K * cin)
+        if (run == 16 && t.bm == 64 && grid <= FF_WK_MAX_WG && g.kpad / FF_KSTEP >= GEN_WK_MIN_STEPS && g.vec >= 4 &&
+            as.M * px_out < 0x100000000ll && (long long)g.kpad * g.cin < 0x100000000ll) {
+            const int rc = ff_wk_generic(as, d, t.bn, s);
+            if (rc != FFK_OK) return rc;
+            continue;
+        }
         if (run == 0) launch_run<0>(t, gd, s, as, g);
         else if (run == 8) launch_run<8>(t, gd, s, as, g);
         else launch_run<16>(t, gd, s, as, g);

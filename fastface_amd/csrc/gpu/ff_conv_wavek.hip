@@ -53,17 +53,21 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 
 constexpr int KW = 8;                                       // waves per workgroup
 
-// A tile of MT x NT 16x16 MFMA blocks: MT*16 pixels, NT*16 channels.
-template <int MT, int NT>
+// A tile of MT*16 pixels and NH column halves (or one) of NT*16 channels:
+// every wave has MT x NT 16x16 MFMA blocks, KG waves share a half's K steps.
+template <int MT, int NT, int NH>
 struct WkTile {
-    static constexpr int BM = MT * 16, BN = NT * 16;
-    static constexpr int PITCH = BN + 4;                    // int32 row pitch of a partial tile
+    static constexpr int BM = MT * 16, BN = NH * NT * 16, KG = KW / NH;
+    static constexpr int PITCH = NT * 16 + 4;               // int32 row pitch of a partial tile
     static constexpr int NTH = KW * 64;
     static constexpr int GROUPS = BM * BN / 4;              // 4 consecutive channels of a pixel each
     static constexpr int GPT = (GROUPS + NTH - 1) / NTH;    // groups per thread
     static constexpr int C4 = BN / 4;                       // groups per pixel
     static constexpr int PART = KW * BM * PITCH * 4;
-    static constexpr int LUT_LD = (BN * FF_LUT_PITCH + 1023) / 1024;
+    // BN tables in LDS; with two halves the partial tiles leave no room, and
+    // the lookups read them from memory
+    static constexpr bool LUT_LDS = NH == 1;
+    static constexpr int LUT_LD = LUT_LDS ? (BN * FF_LUT_PITCH + 1023) / 1024 : 0;
     static_assert(NTH % C4 == 0, "a thread keeps its channels");
 };
 
@@ -101,12 +105,24 @@ __device__ __forceinline__ void wk_pixel(const ConvArgs& a, const WkGeom& g, int
 }
 
 // tap row, tap column and element offset of K step s (a 64-channel run of
-// one tap)
-__device__ __forceinline__ void wk_tap(const WkGeom& g, int s, int& kh, int& kw, int& koff) {
-    const unsigned tap = fdiv((unsigned)s, g.mag_cs);
-    kh = (int)fdiv(tap, g.mag_kw);
-    kw = (int)tap - kh * g.kw;
-    koff = (kh * g.win + kw) * g.cin + (s - (int)tap * g.csteps) * 64;
+// one tap), or, SPAN (channel counts that are multiples of 16 only), of its
+// 16-byte piece q; false past the reduction's end
+template <bool SPAN>
+__device__ __forceinline__ bool wk_tap(const WkGeom& g, int s, int q, int& kh, int& kw, int& koff) {
+    if constexpr (SPAN) {
+        const unsigned k = (unsigned)s * 64 + q * 16;
+        const unsigned tap = fdiv(k, g.mag_cin);
+        kh = (int)fdiv(tap, g.mag_kw);
+        kw = (int)tap - kh * g.kw;
+        koff = (kh * g.win + kw) * g.cin + (int)(k - tap * g.cin);
+        return (int)k < g.ktot;
+    } else {
+        const unsigned tap = fdiv((unsigned)s, g.mag_cs);
+        kh = (int)fdiv(tap, g.mag_kw);
+        kw = (int)tap - kh * g.kw;
+        koff = (kh * g.win + kw) * g.cin + (s - (int)tap * g.csteps) * 64;
+        return true;
+    }
 }
 
 // epilogue operands of a thread's channels, loaded ahead of the reduction
@@ -116,10 +132,10 @@ struct WkEpi {
     int add[GPT];
 };
 
-template <int MT, int NT, bool FC>
-__device__ __forceinline__ void wk_prefetch(const ConvArgs& a, const WkGeom& g, const WkPos& p, WkEpi<WkTile<MT, NT>::GPT>& e,
+template <int MT, int NT, int NH, bool FC>
+__device__ __forceinline__ void wk_prefetch(const ConvArgs& a, const WkGeom& g, const WkPos& p, WkEpi<WkTile<MT, NT, NH>::GPT>& e,
                                             int8_t* lut_s, int wave) {
-    typedef WkTile<MT, NT> T;
+    typedef WkTile<MT, NT, NH> T;
     const int tid = threadIdx.x, lane = tid & 63;
     const int nc = p.n0 + (tid % T::C4) * 4;
     e.ws = e.bias = e.slope = e.adds = e.inv = v4f{0, 0, 0, 0};
@@ -143,7 +159,7 @@ __device__ __forceinline__ void wk_prefetch(const ConvArgs& a, const WkGeom& g, 
                     r_add, (unsigned)(p.m0 + (tid + q * T::NTH) / T::C4) * g.cout + nc, 0, 0);
         }
     }
-    if constexpr (!FC) {
+    if constexpr (!FC && T::LUT_LDS) {
         if ((a.flags & FFK_EPI_BN) && !a.out_i32) {        // BN tables of the tile's channels -> LDS
             constexpr int SPR = FF_LUT_PITCH / 16;
             const __amdgpu_buffer_rsrc_t r_lut = ff_rsrc(a.bn_lut, (unsigned)g.cout * 256);
@@ -162,10 +178,10 @@ __device__ __forceinline__ void wk_prefetch(const ConvArgs& a, const WkGeom& g, 
 }
 
 // partial tiles of the waves -> sums -> (exchange) -> epilogue and stores
-template <int MT, int NT, bool FC>
+template <int MT, int NT, int NH, bool FC>
 __device__ __forceinline__ void wk_finish(const v4i (&acc)[MT][NT], const ConvArgs& a, const WkGeom& g, const WkPos& p,
-                                          const WkEpi<WkTile<MT, NT>::GPT>& ep, int8_t* smem, const int8_t* lut_s, int wave) {
-    typedef WkTile<MT, NT> T;
+                                          const WkEpi<WkTile<MT, NT, NH>::GPT>& ep, int8_t* smem, const int8_t* lut_s, int wave) {
+    typedef WkTile<MT, NT, NH> T;
     constexpr int GPT = T::GPT, GROUPS = T::GROUPS, NTH = T::NTH, C4 = T::C4, PITCH = T::PITCH, BM = T::BM;
     const int tid = threadIdx.x, lane = tid & 63;
     const int lr = lane & 15, lq = lane >> 4;
@@ -187,9 +203,11 @@ __device__ __forceinline__ void wk_finish(const v4i (&acc)[MT][NT], const ConvAr
         const int gi = tid + q * NTH;
         sum[q] = v4i{0, 0, 0, 0};
         if (GROUPS % NTH == 0 || gi < GROUPS) {
-            const int32_t* ps = reinterpret_cast<const int32_t*>(smem) + (gi / C4) * PITCH + c4 * 4;
+            // wave w holds half w % NH of K group w / NH
+            const int half = c4 / (C4 / NH);
+            const int32_t* ps = reinterpret_cast<const int32_t*>(smem) + (half * BM + gi / C4) * PITCH + (c4 - half * (C4 / NH)) * 4;
 #pragma unroll
-            for (int w = 0; w < KW; w++) sum[q] += *reinterpret_cast<const v4i*>(ps + w * BM * PITCH);
+            for (int w = 0; w < T::KG; w++) sum[q] += *reinterpret_cast<const v4i*>(ps + w * NH * BM * PITCH);
         }
     }
     if (FC && g.split > 1) {
@@ -244,6 +262,7 @@ __device__ __forceinline__ void wk_finish(const v4i (&acc)[MT][NT], const ConvAr
     const bool xe = (a.flags & FFK_OUT_X_EVEN) != 0;
     const __amdgpu_buffer_rsrc_t r_x = ff_rsrc(a.out, a.out ? (unsigned)(xe ? a.M / 4 : a.M) * g.cout : 0u);
     const __amdgpu_buffer_rsrc_t r_bn = ff_rsrc(a.out_bn, (a.flags & FFK_EPI_BN) ? (unsigned)a.M * g.cout : 0u);
+    const __amdgpu_buffer_rsrc_t r_lut = ff_rsrc(a.bn_lut, (a.flags & FFK_EPI_BN) ? (unsigned)g.cout * 256 : 0u);
 #pragma unroll
     for (int q = 0; q < GPT; q++) {
         const int gi = tid + q * NTH;
@@ -265,8 +284,10 @@ __device__ __forceinline__ void wk_finish(const v4i (&acc)[MT][NT], const ConvAr
             if (a.flags & FFK_EPI_PRELU) f = ff::prelu(f, ep.slope[e]);
             const int v = ff::requant_haz(f * ep.inv[e]);
             x |= (uint32_t)(uint8_t)v << (8 * e);
-            if (a.flags & FFK_EPI_BN)
-                bn |= (uint32_t)(uint8_t)lut_s[(c4 * 4 + e) * FF_LUT_PITCH + v + 128] << (8 * e);
+            if (a.flags & FFK_EPI_BN) {
+                if constexpr (T::LUT_LDS) bn |= (uint32_t)(uint8_t)lut_s[(c4 * 4 + e) * FF_LUT_PITCH + v + 128] << (8 * e);
+                else bn |= (uint32_t)__builtin_amdgcn_raw_buffer_load_b8(r_lut, (unsigned)((nc + e) * 256 + v + 128), 0, 0) << (8 * e);
+            }
         }
         unsigned xo = (unsigned)m * g.cout + nc;
         if (xe) {
@@ -286,10 +307,12 @@ __device__ __forceinline__ void wk_finish(const v4i (&acc)[MT][NT], const ConvAr
 // whose stages are larger (256->256 @14 at 8 faces: one 4.75 us, two 4.92;
 // more stages were slower everywhere, the eight waves' loads already cover
 // the latency).
-// FC: the head as a 1x1 conv over 1x1 images.
-template <int MT, int NT, int D, bool FC>
+// SPAN: K steps may span taps (wk_tap).  FC: the head as a 1x1 conv over 1x1
+// images.
+template <int MT, int NT, int NH, int D, bool SPAN, bool FC>
 __global__ __launch_bounds__(KW * 64) void conv_wk_kernel(ConvArgs a, WkGeom g) {
-    typedef WkTile<MT, NT> T;
+    typedef WkTile<MT, NT, NH> T;
+    constexpr int KG = T::KG;
     constexpr int LPS = MT + NT, STAGE = LPS * 1024;         // loads per lane, bytes per stage
     constexpr int RING = KW * D * STAGE;
     constexpr int MAIN = RING > T::PART ? RING : T::PART;
@@ -314,20 +337,21 @@ __global__ __launch_bounds__(KW * 64) void conv_wk_kernel(ConvArgs a, WkGeom g) 
             p_base[i] = m < a.M ? m * g.cin + q * 16 : -1;
         } else {
             wk_pixel(a, g, m, p_base[i], p_ih[i], p_iw[i]);
-            p_base[i] += q * 16;
+            if (!SPAN) p_base[i] += q * 16;
         }
     }
     unsigned w_off[NT];
 #pragma unroll
     for (int j = 0; j < NT; j++) {
-        const int n = p.n0 + j * 16 + row;
+        const int n = p.n0 + (wave % NH) * (NT * 16) + j * 16 + row;
         w_off[j] = n < g.cout ? (unsigned)(n * 64 + q * 16) : FF_OOB;
     }
     int8_t* ring = smem + wave * D * STAGE;
-    // this wave's K steps: s_beg + wave + t*KW, t < cnt
-    const int cnt = (p.s_end - p.s_beg - wave + KW - 1) / KW;
+    // this wave's K steps: s_beg + kg + t*KG, t < cnt
+    const int kg = wave / NH;
+    const int cnt = (p.s_end - p.s_beg - kg + KG - 1) / KG;
     auto issue = [&](int t, int slot) {
-        const int s = p.s_beg + wave + t * KW;
+        const int s = p.s_beg + kg + t * KG;
         const unsigned wst = (unsigned)s * (unsigned)(g.cout * 64);
         int8_t* sb = ring + slot * STAGE;
 #pragma unroll
@@ -338,10 +362,10 @@ __global__ __launch_bounds__(KW * 64) void conv_wk_kernel(ConvArgs a, WkGeom g) 
                 bdma16(r_in, p_base[i] >= 0 ? (unsigned)(p_base[i] + s * 64) : FF_OOB, 0, sb + i * 1024);
         } else {
             int kh, kw, koff;
-            wk_tap(g, s, kh, kw, koff);
+            const bool kin = wk_tap<SPAN>(g, s, q, kh, kw, koff);
 #pragma unroll
             for (int i = 0; i < MT; i++) {
-                const bool v = (unsigned)(p_ih[i] + kh) < (unsigned)g.hin && (unsigned)(p_iw[i] + kw) < (unsigned)g.win;
+                const bool v = kin && (unsigned)(p_ih[i] + kh) < (unsigned)g.hin && (unsigned)(p_iw[i] + kw) < (unsigned)g.win;
                 bdma16(r_in, v ? (unsigned)(p_base[i] + koff) : FF_OOB, 0, sb + i * 1024);
             }
         }
@@ -352,7 +376,7 @@ __global__ __launch_bounds__(KW * 64) void conv_wk_kernel(ConvArgs a, WkGeom g) 
 #pragma unroll
         for (int j = 0; j < NT; j++) acc[i][j] = v4i{0, 0, 0, 0};
     WkEpi<T::GPT> ep;
-    wk_prefetch<MT, NT, FC>(a, g, p, ep, lut_s, wave);
+    wk_prefetch<MT, NT, NH, FC>(a, g, p, ep, lut_s, wave);
 #pragma unroll
     for (int u = 0; u < D; u++)
         if (u < cnt) issue(u, u);
@@ -378,7 +402,7 @@ __global__ __launch_bounds__(KW * 64) void conv_wk_kernel(ConvArgs a, WkGeom g) 
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");         // every load into LDS has landed
     __syncthreads();                                         // the rings are free: partial tiles go there
-    wk_finish<MT, NT, FC>(acc, a, g, p, ep, smem, lut_s, wave);
+    wk_finish<MT, NT, NH, FC>(acc, a, g, p, ep, smem, lut_s, wave);
 }
 
 unsigned magic(unsigned d) { return d <= 1 ? 0u : (unsigned)((0x100000000ull + d - 1) / d); }
@@ -397,11 +421,11 @@ int wk_launch(const ConvArgs& a, WkGeom& g, int tile, int split, hipStream_t s) 
     g.mag_split = magic(split);
     const dim3 gd((unsigned)(ff_wk_tiles(tile, a.M, g.cout) * split)), bd(KW * 64);
     switch (tile) {
-    case 0: hipLaunchKernelGGL((conv_wk_kernel<1, 2, 2, FC>), gd, bd, 0, s, a, g); break;
-    case 1: hipLaunchKernelGGL((conv_wk_kernel<2, 2, 2, FC>), gd, bd, 0, s, a, g); break;
-    case 2: hipLaunchKernelGGL((conv_wk_kernel<2, 4, 1, FC>), gd, bd, 0, s, a, g); break;
-    case 3: hipLaunchKernelGGL((conv_wk_kernel<3, 4, 1, FC>), gd, bd, 0, s, a, g); break;
-    default: hipLaunchKernelGGL((conv_wk_kernel<4, 4, 1, FC>), gd, bd, 0, s, a, g); break;
+    case 0: hipLaunchKernelGGL((conv_wk_kernel<1, 2, 1, 2, false, FC>), gd, bd, 0, s, a, g); break;
+    case 1: hipLaunchKernelGGL((conv_wk_kernel<2, 2, 1, 2, false, FC>), gd, bd, 0, s, a, g); break;
+    case 2: hipLaunchKernelGGL((conv_wk_kernel<2, 4, 1, 1, false, FC>), gd, bd, 0, s, a, g); break;
+    case 3: hipLaunchKernelGGL((conv_wk_kernel<3, 4, 1, 1, false, FC>), gd, bd, 0, s, a, g); break;
+    default: hipLaunchKernelGGL((conv_wk_kernel<4, 4, 1, 1, false, FC>), gd, bd, 0, s, a, g); break;
     }
     return ffk_check_launch(FC ? "fc launch" : "conv launch");
 }
@@ -428,7 +452,8 @@ int ff_wk_pick(long long M, int cout, int ksteps, int max_wg) {
     return -1;
 }
 
-int ff_wk_conv(const ConvArgs& a, const ffk_conv_desc* d, int tile, hipStream_t s) {
+namespace {
+WkGeom conv_geom(const ConvArgs& a, const ffk_conv_desc* d) {
     WkGeom g = {};
     g.cin = d->cin; g.cout = d->cout; g.kw = d->kw; g.stride = d->stride; g.pad = d->pad;
     g.hin = d->hin; g.win = d->win;
@@ -436,10 +461,35 @@ int ff_wk_conv(const ConvArgs& a, const ffk_conv_desc* d, int tile, hipStream_t 
     g.wout = (d->win + 2 * d->pad - d->kw) / d->stride + 1;
     g.hw = g.hout * g.wout;
     g.csteps = d->cin / FF_KSTEP;
-    g.ksteps = d->kh * d->kw * g.csteps;
+    g.ktot = d->kh * d->kw * d->cin;
+    g.ksteps = (g.ktot + FF_KSTEP - 1) / FF_KSTEP;
     g.mag_hw = magic(g.hw); g.mag_wo = magic(g.wout); g.mag_kw = magic(d->kw); g.mag_cs = magic(g.csteps);
+    g.mag_cin = magic(g.cin);
     g.in_bytes = (unsigned)((size_t)(a.M / g.hw) * d->hin * d->win * d->cin);
+    return g;
+}
+}  // namespace
+
+int ff_wk_conv(const ConvArgs& a, const ffk_conv_desc* d, int tile, hipStream_t s) {
+    WkGeom g = conv_geom(a, d);
     return wk_launch<false>(a, g, tile, 1, s);
+}
+
+// A conv without a tuned kernel (16-byte channel runs) on 64x64 or 64x128
+// tiles, one per workgroup.
+int ff_wk_generic(const ConvArgs& a, const ffk_conv_desc* d, int bn, hipStream_t s) {
+    WkGeom g = conv_geom(a, d);
+    g.tiles_n = (g.cout + bn - 1) / bn;
+    g.split = 1;
+    g.per_split = g.ksteps;
+    g.mag_tn = magic(g.tiles_n);
+    const dim3 gd((unsigned)(((long long)a.M + 63) / 64 * g.tiles_n)), bd(KW * 64);
+    const bool span = g.cin % FF_KSTEP != 0;
+    if (bn == 64 && span) hipLaunchKernelGGL((conv_wk_kernel<4, 4, 1, 1, true, false>), gd, bd, 0, s, a, g);
+    else if (bn == 64) hipLaunchKernelGGL((conv_wk_kernel<4, 4, 1, 1, false, false>), gd, bd, 0, s, a, g);
+    else if (span) hipLaunchKernelGGL((conv_wk_kernel<4, 4, 2, 1, true, false>), gd, bd, 0, s, a, g);
+    else hipLaunchKernelGGL((conv_wk_kernel<4, 4, 2, 1, false, false>), gd, bd, 0, s, a, g);
+    return ffk_check_launch("generic conv launch");
 }
 
 // The FC head: four K ranges where a tile's grid then fits the CUs, two with

@@ -5,9 +5,9 @@
 
 struct WkGeom {
     int cin, cout, kw, stride, pad, hin, win, hout, wout, hw;
-    int ksteps, csteps;             // 64-byte K steps of the reduction, of one tap
+    int ktot, ksteps, csteps;       // the reduction, its 64-byte K steps, those of one tap
     int tiles_n, split, per_split;  // column tiles, K ranges, steps per range
-    unsigned mag_hw, mag_wo, mag_kw, mag_cs, mag_tn, mag_split;   // divisors' multipliers
+    unsigned mag_hw, mag_wo, mag_kw, mag_cs, mag_cin, mag_tn, mag_split;   // divisors' multipliers
     unsigned in_bytes;
 };
 
@@ -20,6 +20,7 @@ constexpr int FF_WK_MAX_WG_SHARED = 128;
 long long ff_wk_tiles(int tile, long long M, int cout);
 int ff_wk_pick(long long M, int cout, int ksteps, int max_wg);
 int ff_wk_conv(const ConvArgs& a, const ffk_conv_desc* d, int tile, hipStream_t s);
+int ff_wk_generic(const ConvArgs& a, const ffk_conv_desc* d, int bn, hipStream_t s);
 
 struct WkFcPlan { int tile, split; size_t ws_bytes; };
 WkFcPlan ff_wk_fc_plan(int batch, int n, int k, size_t ws_bytes);

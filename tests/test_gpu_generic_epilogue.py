@@ -17,7 +17,11 @@ pytestmark = pytest.mark.gpu
 # tiles of 64 and 128 channels with ragged last blocks, 64 and 128 pixels
 @pytest.mark.parametrize("cin,cout,k,pad,H,B", [
     (32, 16, 3, 1, 9, 2), (32, 80, 3, 1, 9, 2), (16, 136, 1, 0, 12, 3), (24, 104, 3, 1, 10, 2), (48, 36, 3, 1, 9, 2),
-    (20, 100, 3, 1, 9, 2), (7, 5, 3, 1, 10, 2), (16, 131, 3, 1, 8, 2), (32, 128, 1, 0, 60, 10), (48, 60, 3, 1, 58, 12)])
+    (20, 100, 3, 1, 9, 2), (7, 5, 3, 1, 10, 2), (16, 131, 3, 1, 8, 2), (32, 128, 1, 0, 60, 10), (48, 60, 3, 1, 58, 12),
+    # small grids with 12 K steps or more (the wave-split tiles): steps that
+    # span taps and steps of one tap, one and two column halves, ragged ends
+    (80, 64, 3, 1, 9, 3), (48, 100, 5, 2, 11, 2), (16, 72, 7, 3, 8, 1), (128, 36, 3, 1, 9, 2), (192, 260, 3, 0, 9, 2),
+    (112, 128, 3, 1, 37, 11)])
 @pytest.mark.parametrize("offsets", [(0, 0, 0), (8, 8, 8), (16, 4, 0), (0, 16, 1), (3, 0, 16)])
 def test_generic_epilogue_vector_widths(gpu_lib, oracle, cin, cout, k, pad, H, B, offsets):
     lib = gpu_lib
