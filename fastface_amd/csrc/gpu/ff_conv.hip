@@ -78,15 +78,32 @@ struct ConvLaunch {
 // needs more falls back to the whole-K tiling).  FFK_SHARED_GPU: a twin
 // launch runs at the same time, so the large tiles are kept when the two
 // grids together reach FF_MID_MAX_WG.  FFK_LATENCY: the wave-split kernel
-// wherever one of its tiles gives at most a workgroup per CU (ff_wk_pick).
+// wherever one of its tiles gives at most a workgroup per CU (ff_wk_pick),
+// then a tile of the K-group patch kernel that does.
 ConvLaunch choose_launch(const ConvEntry* e, long long M, size_t ws_avail, int flags) {
     const bool shared = (flags & FFK_SHARED_GPU) != 0;
     if ((flags & FFK_LATENCY) && e->cin % FF_KSTEP == 0) {
         const int pad = e->ks / 2, ho = (e->hin + 2 * pad - e->ks) / e->stride + 1;
+        const int lim = shared ? FF_WK_MAX_WG_SHARED : FF_WK_MAX_WG;
         const int t = M * ho * ho > 0xffffffffLL ? -1
-                      : ff_wk_pick(M, e->cout, e->ks * e->ks * (e->cin / FF_KSTEP),
-                                   shared ? FF_WK_MAX_WG_SHARED : FF_WK_MAX_WG);
-        if (t >= 0) return {nullptr, "wavek", e->cout, (int)ff_wk_tiles(t, M, e->cout), 1, 0, 0, t};
+                      : ff_wk_pick(M, e->cout, e->ks * e->ks * (e->cin / FF_KSTEP), lim);
+        // (the patch kernel's 64x64 tiles where there are any)
+        if (t >= 0 && !(t == WK_NTILES - 1 && e->lat[0].fn))
+            return {nullptr, "wavek", e->cout, (int)ff_wk_tiles(t, M, e->cout), 1, 0, 0, t};
+        // The smallest patch tile that gives at most a workgroup per CU, the
+        // 128x128 one included (256->256 @14 at 50 faces, residual+BN: 64x64
+        // tiles of conv_i8_kernel 15.0 us, 128x64 in two rounds 17.0, 128x128
+        // 12.7); the larger ones only where 64-row tiles give more than that
+        // (128->128 @28 at 8 faces: 64x64 6.2 us, 128x64 7.0).
+        if (((M + 63) / 64) * (e->cout / 64) > lim || e->lat[0].fn) {
+            const LatTile tiles[3] = {e->lat[0], e->lat[1],
+                                      {e->lat[1].fn ? e->mid : nullptr, e->mid_bm, e->mid_bn}};
+            for (const LatTile& l : tiles) {
+                if (!l.fn) continue;
+                const long long wgs = ((M + l.bm - 1) / l.bm) * (e->cout / l.bn);
+                if (wgs <= lim) return {l.fn, "patch_kg", l.bn, (int)wgs, 1, 0, 0, -1};
+            }
+        }
     }
     long long big = ((M + e->bm - 1) / e->bm) * (e->cout / e->bn);
     ConvLaunch l = {e->fn, e->kind, e->bn, (int)big, 1, 0, 0, -1};

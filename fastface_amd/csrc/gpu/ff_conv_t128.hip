@@ -10,7 +10,7 @@ const ConvEntry kTable[] = {
     FF_P(64, 128, 56, 1),
     FF_S2(128, 128, 56, FF_S2_SPLIT, 64),
     FF_C128(64, 128, 1, 2, 56, 1),
-    FF_P(128, 128, 28, FF_S2_SPLIT),
+    FF_PL(128, 128, 28, FF_S2_SPLIT, FF_LAT_NONE, FF_LAT_128(128, 128, 28, 2, 2, 2, 2)),
     FF_C128(64, 128, 1, 1, 28, 1),          // shortcut over the compact block input
 };
 }  // namespace

@@ -88,6 +88,13 @@ constexpr int FF_SPLIT_MAX_WG = 320;
 constexpr size_t FF_SPLIT_COUNTER_BYTES = FF_SPLIT_MAX_WG * sizeof(unsigned);
 static_assert(FF_SPLIT_COUNTER_BYTES <= FF_WS_COUNTER_AREA, "counters stay in the reserved area");
 
+// A tile of the K-group patch kernel for the small grids of FFK_LATENCY
+// launches.
+struct LatTile {
+    launch_fn fn;
+    int bm, bn;
+};
+
 struct ConvEntry {
     int cin, cout, ks, stride, hin, win, bm, bn;
     launch_fn fn;
@@ -100,6 +107,7 @@ struct ConvEntry {
     const char* mid_kind;
     int pair_cx;          // stride-2 layers: input channels of the 1x1 shortcut
     launch_pair_fn pair;  // that `fn` runs fused with (conv3s2_shortcut_kernel), or none
+    LatTile lat[2];       // FFK_LATENCY tiles, smaller first (none: no fn)
 };
 
 // A grid of fewer big tiles than this (one per CU) leaves CUs idle; the
@@ -224,10 +232,6 @@ constexpr launch_fn split_launch() {
 #ifndef FF_TPATCH64W
 #define FF_TPATCH64W 8, 1, 2, 2, 4
 #endif
-// Cout >= 256 (stages 3-4)
-#ifndef FF_TPATCH_BIG
-#define FF_TPATCH_BIG FF_TPATCH
-#endif
 #define FF_PENTRY(CIN, COUT, H, SPLIT, MID, WM, WN, MI, NJ, WPE)                      \
     {CIN, COUT, 3, 1, H, H, WM * MI * 32, WN * NJ * 32,                              \
      &launch_patch<CIN, COUT, H, WM, WN, MI, NJ, WPE>, SPLIT,                         \
@@ -235,7 +239,7 @@ constexpr launch_fn split_launch() {
 #define FF_PENTRY_K(CIN, COUT, H, SPLIT, MID, TILE) FF_PENTRY(CIN, COUT, H, SPLIT, MID, TILE)
 #ifdef FF_NO_PATCH
 #define FF_P(CIN, COUT, H, SPLIT) FF_CBIG(CIN, COUT, 3, 1, H, SPLIT)
-#define FF_PB(CIN, COUT, H, SPLIT) FF_CBIG(CIN, COUT, 3, 1, H, SPLIT)
+#define FF_PL(CIN, COUT, H, SPLIT, ...) FF_CBIG(CIN, COUT, 3, 1, H, SPLIT)
 #define FF_P64(CIN, COUT, H, SPLIT) FF_C64(CIN, COUT, 3, 1, H, SPLIT)
 #define FF_P64W(CIN, COUT, H, SPLIT) FF_C64(CIN, COUT, 3, 1, H, SPLIT)
 #else
@@ -267,7 +271,27 @@ constexpr launch_fn split_launch() {
      split_launch<CIN, COUT, 3, 1, H, SPLIT>(), FF_PMID(CIN, COUT, H), "patch", 128, 128, "patch_kg"}
 #define FF_PENTRY_MID_K(CIN, COUT, H, SPLIT, TILE) FF_PENTRY_MID(CIN, COUT, H, SPLIT, TILE)
 #define FF_P(CIN, COUT, H, SPLIT) FF_PENTRY_MID_K(CIN, COUT, H, SPLIT, FF_TPATCH)
-#define FF_PB(CIN, COUT, H, SPLIT) FF_PENTRY_MID_K(CIN, COUT, H, SPLIT, FF_TPATCH_BIG)
+// The same with smaller K-group tiles for the small grids of FFK_LATENCY
+// launches: a CU fetches a tile's input once for all nine taps and its
+// weights once, where 64x64 tiles of nine im2col rows each move half again as
+// much or more (at 64 bytes per clock and CU, 1.9 us of a 256->256 @14
+// launch).  LAT_64 tiles run four K groups of one 64x64 wave, LAT_128 tiles
+// KG groups of two; both step with weights D taps ahead, U taps a barrier.
+// Measured in a graph of 24 launches (us; residual+BN): 256->256 @14 at 19
+// faces 7.2 (wave-split 64x64) -> 6.9 (64x64), at 24 11.0 (64x64 tiles of
+// conv_i8_kernel) -> 8.2 (128x64), at 37 11.2 -> 9.2; 256->512 @14 at 19
+// (PReLU) 11.0 -> 8.1; 128->128 @28 at 19 8.3 -> 7.4; 512->512 @7 at 64
+// 18.6 -> 12.7.
+#define FF_LAT_NONE {nullptr, 0, 0}
+#define FF_LAT_64(CIN, COUT, H) {&launch_patch_kg<CIN, COUT, H, 1, 1, 2, 2, 4, 1, 2, 2>, 64, 64}
+#define FF_LAT_128(CIN, COUT, H, KG, WPE, D, U) {&launch_patch_kg<CIN, COUT, H, 2, 1, 2, 2, KG, WPE, D, U>, 128, 64}
+#define FF_PL_TILE(CIN, COUT, H, SPLIT, WM, WN, MI, NJ, WPE, ...)                    \
+    {CIN, COUT, 3, 1, H, H, WM * MI * 32, WN * NJ * 32,                              \
+     &launch_patch<CIN, COUT, H, WM, WN, MI, NJ, WPE>, SPLIT,                         \
+     split_launch<CIN, COUT, 3, 1, H, SPLIT>(), FF_PMID(CIN, COUT, H), "patch", 128, 128, "patch_kg", \
+     0, nullptr, {__VA_ARGS__}}
+#define FF_PL_K(CIN, COUT, H, SPLIT, ...) FF_PL_TILE(CIN, COUT, H, SPLIT, __VA_ARGS__)
+#define FF_PL(CIN, COUT, H, SPLIT, ...) FF_PL_K(CIN, COUT, H, SPLIT, FF_TPATCH, __VA_ARGS__)
 #define FF_P64(CIN, COUT, H, SPLIT) FF_PENTRY_K(CIN, COUT, H, SPLIT, nullptr, FF_TPATCH64)
 // (small grids: the 256x64 tiles, twice the workgroups)
 #define FF_P64W(CIN, COUT, H, SPLIT)                                                \

@@ -122,8 +122,9 @@ typedef struct { const float* in; float* out; } ffk_io;
                                    the launch is one of a chain in which each
                                    waits for the one before, so a small grid
                                    is tiled for the shortest single launch
-                                   ("wavek", ffk_conv_variant), which needs
-                                   no workspace.  No reference counterpart. */
+                                   ("wavek" or "patch_kg", ffk_conv_variant),
+                                   which needs no workspace.  No reference
+                                   counterpart. */
 
 /* rows of the per-layer parameter block, each `cout` floats (device) */
 enum {

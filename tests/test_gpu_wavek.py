@@ -20,7 +20,21 @@ CASES = [
     (256, 256, 3, 1, 14, 5, 31 * 8), (64, 64, 3, 2, 112, 1, 98 * 2),                       # 32x32
     (256, 256, 3, 1, 14, 8, 49 * 4), (64, 128, 3, 1, 56, 1, 98 * 2), (256, 256, 3, 2, 28, 10, 62 * 4),   # 32x64
     (256, 256, 3, 1, 14, 11, 45 * 4), (512, 512, 3, 2, 14, 31, 32 * 8),                    # 48x64
-    (256, 256, 3, 1, 14, 17, 53 * 4), (512, 512, 3, 1, 7, 41, 32 * 8),                     # 64x64
+    (256, 256, 3, 2, 28, 17, 53 * 4), (512, 512, 3, 1, 7, 41, 32 * 8),                     # 64x64
+]
+
+# the K-group patch kernel's tiles past those, at the first and last batch
+# each one takes (64x64, 128x64, then 128x128), also as one of two halves
+SH = fa.FFK_SHARED_GPU
+PATCH_CASES = [
+    (256, 256, 3, 1, 14, 16, 49 * 4, 0), (256, 256, 3, 1, 14, 20, 62 * 4, 0),
+    (256, 256, 3, 1, 14, 21, 33 * 4, 0), (256, 256, 3, 1, 14, 41, 63 * 4, 0), (256, 256, 3, 1, 14, 42, 65 * 2, 0),
+    (256, 256, 3, 1, 14, 20, 31 * 4, SH), (256, 256, 3, 1, 14, 10, 31 * 4, SH),
+    (256, 512, 3, 1, 14, 8, 25 * 8, 0), (256, 512, 3, 1, 14, 10, 31 * 8, 0),
+    (256, 512, 3, 1, 14, 11, 17 * 8, 0), (256, 512, 3, 1, 14, 20, 31 * 8, 0),
+    (128, 128, 3, 1, 28, 11, 68 * 2, 0), (128, 128, 3, 1, 28, 20, 123 * 2, 0), (128, 128, 3, 1, 28, 21, 129, 0),
+    (128, 256, 3, 1, 28, 6, 37 * 4, 0), (128, 256, 3, 1, 28, 10, 62 * 4, 0),
+    (512, 512, 3, 1, 7, 42, 17 * 8, 0), (512, 512, 3, 1, 7, 83, 32 * 8, 0),
 ]
 
 
@@ -34,8 +48,17 @@ def _desc(cin, cout, k, s, H, B, flags):
 @pytest.mark.parametrize("mode", ["raw", "all", "bn_only", "inscale"])
 @pytest.mark.parametrize("cin,cout,k,s,H,B,grid", CASES)
 def test_wavek_conv(gpu_lib, oracle, cin, cout, k, s, H, B, grid, mode):
-    lib, L = gpu_lib, fa.FFK_LATENCY
-    assert lib.ffk_conv_variant(_desc(cin, cout, k, s, H, B, L)) == b"wavek"
+    _check_conv(gpu_lib, oracle, cin, cout, k, s, H, B, grid, mode, fa.FFK_LATENCY, b"wavek")
+
+
+@pytest.mark.parametrize("mode", ["raw", "all"])
+@pytest.mark.parametrize("cin,cout,k,s,H,B,grid,shared", PATCH_CASES)
+def test_latency_patch_tiles(gpu_lib, oracle, cin, cout, k, s, H, B, grid, shared, mode):
+    _check_conv(gpu_lib, oracle, cin, cout, k, s, H, B, grid, mode, fa.FFK_LATENCY | shared, b"patch_kg")
+
+
+def _check_conv(lib, oracle, cin, cout, k, s, H, B, grid, mode, L, kind):
+    assert lib.ffk_conv_variant(_desc(cin, cout, k, s, H, B, L)) == kind
     assert lib.ffk_conv_grid(_desc(cin, cout, k, s, H, B, L)) == grid
     assert lib.ffk_conv_workspace_bytes(_desc(cin, cout, k, s, H, B, L)) == 0
     r = rng(3100 + cin + cout + k + H + B)
