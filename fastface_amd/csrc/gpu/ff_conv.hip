@@ -449,16 +449,28 @@ int ffk_conv_s2_shortcut(const ffk_conv_desc* c, const ffk_conv_desc* s, void* s
     if ((s->flags & FFK_EPI_BN) ? (!s->out_bn || !s->bn_lut) : !s->out) return 0;
     if ((s->flags & FFK_OUT_X_EVEN) && ((ho & 1) || !s->out)) return 0;
     const ConvEntry* e = find_conv(c->cin, c->cout, 3, 3, 2, 1, c->hin, c->win);
-    if (!e || !e->pair || e->pair_cx != s->cin) return 0;
+    if (!e) return 0;
     const long long M = conv_pixels(c);
     if (M == 0) return 1;
     // one launch over the whole batch: every tensor below 2 GiB
     const long long lim = 0x7fffffffLL;
     if ((long long)c->batch * c->hin * c->win * c->cin > lim || M * c->cout > lim || M * s->cin > lim) return 0;
-    const ConvLaunch l = choose_launch(e, M, c->workspace ? c->workspace_bytes : 0, c->flags);
-    if (l.fn != e->fn) return 0;
     ConvArgs a = conv_args(c), b = conv_args(s);
     a.M = b.M = (int)M;
+    // a small grid of a chain: the wave-split kernel (the shortcut's K steps
+    // go to different waves, so at most eight)
+    if ((c->flags & s->flags & FFK_LATENCY) && c->cin % FF_KSTEP == 0 && s->cin % FF_KSTEP == 0 &&
+        s->cin <= 8 * FF_KSTEP && M * ho * ho <= 0xffffffffLL && find_conv(s->cin, s->cout, 1, 1, 1, 0, ho, ho)) {
+        const int t = ff_wk_pick(M, c->cout, 9 * (c->cin / FF_KSTEP),
+                                 (c->flags & FFK_SHARED_GPU) ? FF_WK_MAX_WG_SHARED : FF_WK_MAX_WG);
+        if (t >= 0 && t < WK_NTILES - 1) {
+            const int rc = ff_wk_pair(a, b, c, s, t, (hipStream_t)stream);
+            return rc != FFK_OK ? rc : 1;
+        }
+    }
+    if (!e->pair || e->pair_cx != s->cin) return 0;
+    const ConvLaunch l = choose_launch(e, M, c->workspace ? c->workspace_bytes : 0, c->flags);
+    if (l.fn != e->fn) return 0;
     a.tiles_n = b.tiles_n = c->cout / l.bn;
     e->pair(a, b, l.grid, (hipStream_t)stream);
     const int rc = ffk_check_launch("conv pair launch");

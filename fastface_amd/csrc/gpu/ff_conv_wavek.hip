@@ -125,6 +125,18 @@ __device__ __forceinline__ bool wk_tap(const WkGeom& g, int s, int q, int& kh, i
     }
 }
 
+// The second conv of a launch: none, or the 1x1 shortcut (over the compact
+// block input, csteps K steps, at most one a wave) that adds the first's
+// int8 result (ffk_conv_s2_shortcut).
+struct WkOne {
+    static constexpr bool PAIR = false;
+};
+struct WkPair {
+    static constexpr bool PAIR = true;
+    ConvArgs b;
+    int cin, csteps;
+};
+
 // epilogue operands of a thread's channels, loaded ahead of the reduction
 template <int GPT>
 struct WkEpi {
@@ -132,7 +144,7 @@ struct WkEpi {
     int add[GPT];
 };
 
-template <int MT, int NT, int NH, bool FC>
+template <int MT, int NT, int NH, bool FC, bool PAIR>
 __device__ __forceinline__ void wk_prefetch(const ConvArgs& a, const WkGeom& g, const WkPos& p, WkEpi<WkTile<MT, NT, NH>::GPT>& e,
                                             int8_t* lut_s, int wave) {
     typedef WkTile<MT, NT, NH> T;
@@ -150,8 +162,8 @@ __device__ __forceinline__ void wk_prefetch(const ConvArgs& a, const WkGeom& g, 
         e.bias = *reinterpret_cast<const v4f*>(P + FFK_P_BIAS * g.cout);
         e.inv = *reinterpret_cast<const v4f*>(P + FFK_P_INV * g.cout);
         if (a.flags & FFK_EPI_PRELU) e.slope = *reinterpret_cast<const v4f*>(P + FFK_P_SLOPE * g.cout);
-        if (a.flags & FFK_EPI_ADD) {
-            e.adds = *reinterpret_cast<const v4f*>(P + FFK_P_ADDSCALE * g.cout);
+        if (a.flags & FFK_EPI_ADD) e.adds = *reinterpret_cast<const v4f*>(P + FFK_P_ADDSCALE * g.cout);
+        if ((a.flags & FFK_EPI_ADD) && !PAIR) {            // (a pair's residual is its own first result)
             const __amdgpu_buffer_rsrc_t r_add = ff_rsrc(a.add_src, (unsigned)a.M * g.cout);
 #pragma unroll
             for (int q = 0; q < T::GPT; q++)
@@ -177,10 +189,13 @@ __device__ __forceinline__ void wk_prefetch(const ConvArgs& a, const WkGeom& g, 
     }
 }
 
-// partial tiles of the waves -> sums -> (exchange) -> epilogue and stores
-template <int MT, int NT, int NH, bool FC>
+// Partial tiles of the waves -> sums -> (exchange) -> epilogue and stores.
+// A pair: `a` is the shortcut, `first` the first conv, `acc2` the shortcut's
+// partial of the waves that took one of its K steps (`mine` >= 0).
+template <int MT, int NT, int NH, bool FC, typename X>
 __device__ __forceinline__ void wk_finish(const v4i (&acc)[MT][NT], const ConvArgs& a, const WkGeom& g, const WkPos& p,
-                                          const WkEpi<WkTile<MT, NT, NH>::GPT>& ep, int8_t* smem, const int8_t* lut_s, int wave) {
+                                          const WkEpi<WkTile<MT, NT, NH>::GPT>& ep, int8_t* smem, const int8_t* lut_s, int wave,
+                                          const ConvArgs& first, const X& x2, const v4i (&acc2)[MT][NT], int mine) {
     typedef WkTile<MT, NT, NH> T;
     constexpr int GPT = T::GPT, GROUPS = T::GROUPS, NTH = T::NTH, C4 = T::C4, PITCH = T::PITCH, BM = T::BM;
     const int tid = threadIdx.x, lane = tid & 63;
@@ -198,6 +213,9 @@ __device__ __forceinline__ void wk_finish(const v4i (&acc)[MT][NT], const ConvAr
     }
     __syncthreads();
     v4i sum[GPT];
+    int resid[GPT];
+#pragma unroll
+    for (int q = 0; q < GPT; q++) resid[q] = X::PAIR ? 0 : ep.add[q];
 #pragma unroll
     for (int q = 0; q < GPT; q++) {
         const int gi = tid + q * NTH;
@@ -208,6 +226,41 @@ __device__ __forceinline__ void wk_finish(const v4i (&acc)[MT][NT], const ConvAr
             const int32_t* ps = reinterpret_cast<const int32_t*>(smem) + (half * BM + gi / C4) * PITCH + (c4 - half * (C4 / NH)) * 4;
 #pragma unroll
             for (int w = 0; w < T::KG; w++) sum[q] += *reinterpret_cast<const v4i*>(ps + w * NH * BM * PITCH);
+        }
+    }
+    if constexpr (X::PAIR) {
+        // the first conv's int8 results, then the shortcut's sums
+        v4f ws = {}, bias = {}, inv = {};
+        if (nok) {
+            ws = *reinterpret_cast<const v4f*>(first.params + FFK_P_WS * g.cout + nc);
+            bias = *reinterpret_cast<const v4f*>(first.params + FFK_P_BIAS * g.cout + nc);
+            inv = *reinterpret_cast<const v4f*>(first.params + FFK_P_INV * g.cout + nc);
+        }
+        __syncthreads();                                     // the first partial tiles are read
+        int32_t* ps = reinterpret_cast<int32_t*>(smem);
+        if (mine >= 0)
+#pragma unroll
+            for (int i = 0; i < MT; i++)
+#pragma unroll
+                for (int j = 0; j < NT; j++)
+                    *reinterpret_cast<v4i*>(ps + (mine * BM + i * 16 + lr) * PITCH + j * 16 + lq * 4) = acc2[i][j];
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < GPT; q++) {
+            const int gi = tid + q * NTH;
+            uint32_t v = 0;
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                float f = (float)sum[q][e];
+                f = f * ws[e];
+                f = f + bias[e];
+                v |= (uint32_t)(uint8_t)ff::requant_haz(f * inv[e]) << (8 * e);
+            }
+            resid[q] = (int)v;
+            sum[q] = v4i{0, 0, 0, 0};
+            if (GROUPS % NTH == 0 || gi < GROUPS)
+                for (int w = 0; w < x2.csteps; w++)
+                    sum[q] += *reinterpret_cast<const v4i*>(ps + (w * BM + gi / C4) * PITCH + c4 * 4);
         }
     }
     if (FC && g.split > 1) {
@@ -280,7 +333,7 @@ __device__ __forceinline__ void wk_finish(const v4i (&acc)[MT][NT], const ConvAr
             if (a.flags & FFK_EPI_INSCALE) f = f * a.in_scale;
             f = f * ep.ws[e];
             f = f + ep.bias[e];
-            if (a.flags & FFK_EPI_ADD) f = ff::add_residual(f, (int32_t)(int8_t)((uint32_t)ep.add[q] >> (8 * e)), ep.adds[e]);
+            if (a.flags & FFK_EPI_ADD) f = ff::add_residual(f, (int32_t)(int8_t)((uint32_t)resid[q] >> (8 * e)), ep.adds[e]);
             if (a.flags & FFK_EPI_PRELU) f = ff::prelu(f, ep.slope[e]);
             const int v = ff::requant_haz(f * ep.inv[e]);
             x |= (uint32_t)(uint8_t)v << (8 * e);
@@ -309,8 +362,9 @@ __device__ __forceinline__ void wk_finish(const v4i (&acc)[MT][NT], const ConvAr
 // the latency).
 // SPAN: K steps may span taps (wk_tap).  FC: the head as a 1x1 conv over 1x1
 // images.
-template <int MT, int NT, int NH, int D, bool SPAN, bool FC>
-__global__ __launch_bounds__(KW * 64) void conv_wk_kernel(ConvArgs a, WkGeom g) {
+// X: WkPair, or one conv.
+template <int MT, int NT, int NH, int D, bool SPAN, bool FC, typename X>
+__global__ __launch_bounds__(KW * 64) void conv_wk_kernel(ConvArgs a, WkGeom g, X x2) {
     typedef WkTile<MT, NT, NH> T;
     constexpr int KG = T::KG;
     constexpr int LPS = MT + NT, STAGE = LPS * 1024;         // loads per lane, bytes per stage
@@ -349,9 +403,29 @@ __global__ __launch_bounds__(KW * 64) void conv_wk_kernel(ConvArgs a, WkGeom g) 
     int8_t* ring = smem + wave * D * STAGE;
     // this wave's K steps: s_beg + kg + t*KG, t < cnt
     const int kg = wave / NH;
-    const int cnt = (p.s_end - p.s_beg - kg + KG - 1) / KG;
+    const int main_cnt = (p.s_end - p.s_beg - kg + KG - 1) / KG;
+    int cnt = main_cnt, mine = -1;
+    if constexpr (X::PAIR) {
+        // the shortcut's steps follow the first conv's in the same order: the
+        // waves after its last step take them, as their last
+        const int i = (kg - p.s_end) & (KG - 1);
+        if (i < x2.csteps) { mine = i; cnt++; }
+    }
     auto issue = [&](int t, int slot) {
         const int s = p.s_beg + kg + t * KG;
+        if constexpr (X::PAIR) {
+            if (t == main_cnt) {
+                const __amdgpu_buffer_rsrc_t r_in2 = ff_rsrc(x2.b.in, (unsigned)a.M * x2.cin);
+                const __amdgpu_buffer_rsrc_t r_w2 = ff_rsrc(x2.b.w, (unsigned)x2.csteps * g.cout * 64);
+                int8_t* sb = ring + slot * STAGE;
+#pragma unroll
+                for (int j = 0; j < NT; j++) bdma16(r_w2, w_off[j], (unsigned)mine * (unsigned)(g.cout * 64), sb + (MT + j) * 1024);
+#pragma unroll
+                for (int i = 0; i < MT; i++)
+                    bdma16(r_in2, (unsigned)((p.m0 + i * 16 + row) * x2.cin + mine * 64 + q * 16), 0, sb + i * 1024);
+                return;
+            }
+        }
         const unsigned wst = (unsigned)s * (unsigned)(g.cout * 64);
         int8_t* sb = ring + slot * STAGE;
 #pragma unroll
@@ -370,13 +444,17 @@ __global__ __launch_bounds__(KW * 64) void conv_wk_kernel(ConvArgs a, WkGeom g) 
             }
         }
     };
-    v4i acc[MT][NT];
+    v4i acc[MT][NT], acc2[MT][NT];
 #pragma unroll
     for (int i = 0; i < MT; i++)
 #pragma unroll
-        for (int j = 0; j < NT; j++) acc[i][j] = v4i{0, 0, 0, 0};
+        for (int j = 0; j < NT; j++) acc[i][j] = acc2[i][j] = v4i{0, 0, 0, 0};
     WkEpi<T::GPT> ep;
-    wk_prefetch<MT, NT, NH, FC>(a, g, p, ep, lut_s, wave);
+    const ConvArgs& last = [&]() -> const ConvArgs& {
+        if constexpr (X::PAIR) return x2.b;
+        else return a;
+    }();
+    wk_prefetch<MT, NT, NH, FC, X::PAIR>(last, g, p, ep, lut_s, wave);
 #pragma unroll
     for (int u = 0; u < D; u++)
         if (u < cnt) issue(u, u);
@@ -393,16 +471,24 @@ __global__ __launch_bounds__(KW * 64) void conv_wk_kernel(ConvArgs a, WkGeom g) 
         for (int j = 0; j < NT; j++) fw[j] = *reinterpret_cast<const v4i*>(sb + (MT + j) * 1024);
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the stage is read: its slot is free
         if (t + D < cnt) issue(t + D, slot);
+        if (X::PAIR && t == main_cnt) {
 #pragma unroll
-        for (int i = 0; i < MT; i++)
+            for (int i = 0; i < MT; i++)
 #pragma unroll
-            for (int j = 0; j < NT; j++)
-                acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fw[j], fp[i], acc[i][j], 0, 0, 0);
+                for (int j = 0; j < NT; j++)
+                    acc2[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fw[j], fp[i], acc2[i][j], 0, 0, 0);
+        } else {
+#pragma unroll
+            for (int i = 0; i < MT; i++)
+#pragma unroll
+                for (int j = 0; j < NT; j++)
+                    acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fw[j], fp[i], acc[i][j], 0, 0, 0);
+        }
         slot = slot + 1 == D ? 0 : slot + 1;
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");         // every load into LDS has landed
     __syncthreads();                                         // the rings are free: partial tiles go there
-    wk_finish<MT, NT, NH, FC>(acc, a, g, p, ep, smem, lut_s, wave);
+    wk_finish<MT, NT, NH, FC>(acc, last, g, p, ep, smem, lut_s, wave, a, x2, acc2, mine);
 }
 
 unsigned magic(unsigned d) { return d <= 1 ? 0u : (unsigned)((0x100000000ull + d - 1) / d); }
@@ -411,8 +497,8 @@ unsigned magic(unsigned d) { return d <= 1 ? 0u : (unsigned)((0x100000000ull + d
 struct WkTileSize { int bm, bn; };
 constexpr WkTileSize WK_TILES[WK_NTILES] = {{16, 32}, {32, 32}, {32, 64}, {48, 64}, {64, 64}};
 
-template <bool FC>
-int wk_launch(const ConvArgs& a, WkGeom& g, int tile, int split, hipStream_t s) {
+template <bool FC, typename X>
+int wk_launch(const ConvArgs& a, WkGeom& g, int tile, int split, hipStream_t s, const X& x) {
     const WkTileSize& ts = WK_TILES[tile];
     g.tiles_n = (g.cout + ts.bn - 1) / ts.bn;
     g.split = split;
@@ -421,11 +507,14 @@ int wk_launch(const ConvArgs& a, WkGeom& g, int tile, int split, hipStream_t s) 
     g.mag_split = magic(split);
     const dim3 gd((unsigned)(ff_wk_tiles(tile, a.M, g.cout) * split)), bd(KW * 64);
     switch (tile) {
-    case 0: hipLaunchKernelGGL((conv_wk_kernel<1, 2, 1, 2, false, FC>), gd, bd, 0, s, a, g); break;
-    case 1: hipLaunchKernelGGL((conv_wk_kernel<2, 2, 1, 2, false, FC>), gd, bd, 0, s, a, g); break;
-    case 2: hipLaunchKernelGGL((conv_wk_kernel<2, 4, 1, 1, false, FC>), gd, bd, 0, s, a, g); break;
-    case 3: hipLaunchKernelGGL((conv_wk_kernel<3, 4, 1, 1, false, FC>), gd, bd, 0, s, a, g); break;
-    default: hipLaunchKernelGGL((conv_wk_kernel<4, 4, 1, 1, false, FC>), gd, bd, 0, s, a, g); break;
+    case 0: hipLaunchKernelGGL((conv_wk_kernel<1, 2, 1, 2, false, FC, X>), gd, bd, 0, s, a, g, x); break;
+    case 1: hipLaunchKernelGGL((conv_wk_kernel<2, 2, 1, 2, false, FC, X>), gd, bd, 0, s, a, g, x); break;
+    case 2: hipLaunchKernelGGL((conv_wk_kernel<2, 4, 1, 1, false, FC, X>), gd, bd, 0, s, a, g, x); break;
+    case 3: hipLaunchKernelGGL((conv_wk_kernel<3, 4, 1, 1, false, FC, X>), gd, bd, 0, s, a, g, x); break;
+    default:
+        // (a pair's second accumulators do not fit a 64x64 tile's registers)
+        if constexpr (!X::PAIR) hipLaunchKernelGGL((conv_wk_kernel<4, 4, 1, 1, false, FC, X>), gd, bd, 0, s, a, g, x);
+        break;
     }
     return ffk_check_launch(FC ? "fc launch" : "conv launch");
 }
@@ -472,7 +561,18 @@ WkGeom conv_geom(const ConvArgs& a, const ffk_conv_desc* d) {
 
 int ff_wk_conv(const ConvArgs& a, const ffk_conv_desc* d, int tile, hipStream_t s) {
     WkGeom g = conv_geom(a, d);
-    return wk_launch<false>(a, g, tile, 1, s);
+    return wk_launch<false>(a, g, tile, 1, s, WkOne{});
+}
+
+// A stride-2 conv and the 1x1 shortcut that adds its result, as one launch:
+// the launch saved (3 to 5 us in a
+// chain) outweighs the shortcut's few K steps and a second exchange of partial
+// tiles.  Measured on whole calls: 1 face 250 -> 240 us (four pairs), 8 faces
+// 372 -> 364 (two), 20 faces 484 -> 479.
+int ff_wk_pair(const ConvArgs& a, const ConvArgs& b, const ffk_conv_desc* c, const ffk_conv_desc* sc, int tile,
+               hipStream_t s) {
+    WkGeom g = conv_geom(a, c);
+    return wk_launch<false>(a, g, tile, 1, s, WkPair{b, sc->cin, sc->cin / FF_KSTEP});
 }
 
 // A conv without a tuned kernel (16-byte channel runs) on 64x64 or 64x128
@@ -485,10 +585,10 @@ int ff_wk_generic(const ConvArgs& a, const ffk_conv_desc* d, int bn, hipStream_t
     g.mag_tn = magic(g.tiles_n);
     const dim3 gd((unsigned)(((long long)a.M + 63) / 64 * g.tiles_n)), bd(KW * 64);
     const bool span = g.cin % FF_KSTEP != 0;
-    if (bn == 64 && span) hipLaunchKernelGGL((conv_wk_kernel<4, 4, 1, 1, true, false>), gd, bd, 0, s, a, g);
-    else if (bn == 64) hipLaunchKernelGGL((conv_wk_kernel<4, 4, 1, 1, false, false>), gd, bd, 0, s, a, g);
-    else if (span) hipLaunchKernelGGL((conv_wk_kernel<4, 4, 2, 1, true, false>), gd, bd, 0, s, a, g);
-    else hipLaunchKernelGGL((conv_wk_kernel<4, 4, 2, 1, false, false>), gd, bd, 0, s, a, g);
+    if (bn == 64 && span) hipLaunchKernelGGL((conv_wk_kernel<4, 4, 1, 1, true, false, WkOne>), gd, bd, 0, s, a, g, WkOne{});
+    else if (bn == 64) hipLaunchKernelGGL((conv_wk_kernel<4, 4, 1, 1, false, false, WkOne>), gd, bd, 0, s, a, g, WkOne{});
+    else if (span) hipLaunchKernelGGL((conv_wk_kernel<4, 4, 2, 1, true, false, WkOne>), gd, bd, 0, s, a, g, WkOne{});
+    else hipLaunchKernelGGL((conv_wk_kernel<4, 4, 2, 1, false, false, WkOne>), gd, bd, 0, s, a, g, WkOne{});
     return ffk_check_launch("generic conv launch");
 }
 
@@ -530,5 +630,5 @@ int ff_wk_fc(const ffk_fc_desc* d, hipStream_t s) {
     g.cin = d->k; g.cout = d->n;
     g.ksteps = d->k / FF_KSTEP;
     g.in_bytes = (unsigned)((size_t)d->batch * d->k);
-    return wk_launch<true>(a, g, p.tile, p.split, s);
+    return wk_launch<true>(a, g, p.tile, p.split, s, WkOne{});
 }

@@ -20,6 +20,8 @@ constexpr int FF_WK_MAX_WG_SHARED = 128;
 long long ff_wk_tiles(int tile, long long M, int cout);
 int ff_wk_pick(long long M, int cout, int ksteps, int max_wg);
 int ff_wk_conv(const ConvArgs& a, const ffk_conv_desc* d, int tile, hipStream_t s);
+int ff_wk_pair(const ConvArgs& a, const ConvArgs& b, const ffk_conv_desc* c, const ffk_conv_desc* sc, int tile,
+               hipStream_t s);
 int ff_wk_generic(const ConvArgs& a, const ffk_conv_desc* d, int bn, hipStream_t s);
 
 struct WkFcPlan { int tile, split; size_t ws_bytes; };

@@ -7,8 +7,9 @@ import numpy as np
 import pytest
 
 import fastface_amd as fa
+import gpu_util
 from gpu_util import params_block, run_conv, run_fc
-from test_gpu_kernels import F32, _special_params, rng
+from test_gpu_kernels import F32, _pair_desc, _special_params, rng
 
 pytestmark = pytest.mark.gpu
 
@@ -126,3 +127,57 @@ def test_wavek_fc_other_heads(gpu_lib, oracle, B, K, N, split):
     got = run_fc(gpu_lib, a, W, ws, bias, split=split)
     for b in range(B):
         assert np.array_equal(got[b], oracle.fc(a[b], W, ws, bias)), b
+
+
+# (cin, cout, H, shortcut's cin, batch): a stride-2 conv and its shortcut as
+# one launch, on every tile it takes, ragged last row tiles, one to four
+# shortcut steps, the first conv's steps a multiple of the waves or not
+PAIRS = [(64, 64, 112, 64, 1), (128, 128, 56, 64, 1), (128, 128, 56, 64, 2), (256, 256, 28, 128, 1), (256, 256, 28, 128, 7),
+         (256, 256, 28, 128, 13), (512, 512, 14, 256, 1), (512, 512, 14, 256, 9), (512, 512, 14, 256, 31)]
+
+
+@pytest.mark.parametrize("form", ["x_bn", "x", "bn", "x_even"])
+@pytest.mark.parametrize("cin,cout,H,cx,B", PAIRS)
+def test_wavek_pair_equals_two_launches(gpu_lib, cin, cout, H, cx, B, form):
+    lib, L = gpu_lib, fa.FFK_LATENCY
+    Ho = H // 2
+    if form == "x_even" and Ho % 2:
+        pytest.skip("odd output image")
+    r = rng(3400 + cin + H + B)
+    x = r.integers(-128, 128, size=(B, H, H, cin), dtype=np.int8)
+    w = r.integers(-128, 128, size=(cout, cin, 3, 3), dtype=np.int8)
+    xc = r.integers(-128, 128, size=(B, Ho, Ho, cx), dtype=np.int8)
+    w2 = r.integers(-128, 128, size=(cout, cx, 1, 1), dtype=np.int8)
+    x[0] = -128
+    w[-1] = -128
+    ws, bias, inv = _special_params(r, cout)
+    P1 = params_block(cout, ws=ws, bias=bias, inv=inv)
+    ws2, bias2, inv2 = _special_params(r, cout)
+    P2 = params_block(cout, ws=ws2, bias=bias2, inv=inv2, adds=r.uniform(1e-3, 5e-2, cout).astype(F32),
+                      bn_sin=r.uniform(1e-3, 5e-2, cout).astype(F32), bn_s=r.uniform(0.5, 1.5, cout).astype(F32),
+                      bn_o=r.normal(0, 0.05, cout).astype(F32), bn_inv=(1.0 / r.uniform(0.01, 0.1, cout)).astype(F32))
+    want_bn = form != "x"
+    f1 = fa.FFK_EPI_BIAS
+    f2 = fa.FFK_EPI_BIAS | fa.FFK_EPI_ADD | (fa.FFK_EPI_BN if want_bn else 0)
+    R, _ = run_conv(lib, x, w, 2, 1, params=P1, flags=f1, split=False)
+    X_exp, BN_exp = run_conv(lib, xc, w2, 1, 0, params=P2, flags=f2, add=R, want_bn=want_bn, split=False)
+
+    keep = []
+    n = B * Ho * Ho * cout
+    dR, dX, dBN = (gpu_util.Dev(lib, host=np.full(n, 0x5A, np.uint8)) for _ in range(3))
+    keep += [dR, dX, dBN]
+    c = _pair_desc(lib, keep, B, cin, cout, 3, 2, 1, H, x, w, P1, f1 | L, dR.ptr)
+    sc = _pair_desc(lib, keep, B, cx, cout, 1, 1, 0, Ho, xc, w2, P2,
+                    f2 | L | (fa.FFK_OUT_X_EVEN if form == "x_even" else 0), None if form == "bn" else dX.ptr,
+                    out_bn=dBN.ptr if want_bn else None, add=dR.ptr)
+    assert lib.ffk_conv_s2_shortcut(C.byref(c), C.byref(sc), None) == 1
+    gpu_util.check(lib, lib.ffk_stream_sync(None))
+    X = dX.get(np.int8, (n,))
+    if form == "x_even":
+        ne = n // 4
+        assert np.array_equal(X[:ne].reshape(B, Ho // 2, Ho // 2, cout), X_exp[:, ::2, ::2])
+        assert (X[ne:].view(np.uint8) == 0x5A).all()
+    elif form != "bn":
+        assert np.array_equal(X.reshape(X_exp.shape), X_exp)
+    if want_bn:
+        assert np.array_equal(dBN.get(np.int8, BN_exp.shape), BN_exp)
