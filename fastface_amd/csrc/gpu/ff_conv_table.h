@@ -77,7 +77,8 @@ constexpr int FF_SPLIT_MAX_WG = 320;
 // a batch run at once (FFK_SHARED_GPU).  Measured on the chain at 1-64 faces
 // with limits 0, 200, 320 and 640: 640 is fastest at 8 and 16 faces (8:
 // 0.524 ms without these tiles, 0.486 with), 200 at the 48- and 64-face
-// halves; b=1 takes them for every layer without a split (0.399 -> 0.374 ms).
+// halves; b=1 took them for every layer without a split (0.399 -> 0.374 ms)
+// before FFK_LATENCY launches had smaller tiles.
 #ifndef FF_TILE64_MAX_WG
 #define FF_TILE64_MAX_WG 640
 #endif

@@ -26,7 +26,9 @@
  * <geometry> <flags>", or "... map|add <channels> <pixels>" for a
  * stand-alone BN / PReLU / Add), built as fastface.c builds its descriptors (two
  * halves from 24 faces, FFK_SHARED_GPU) from the library's host-side
- * launch choice: no device is involved. */
+ * launch choice: no device is involved.  The convs are listed as a caller
+ * without the chain's FFK_LATENCY hint gets them; an fc line names the
+ * batch's size class (up to 16 faces "matvec"). */
 #include <stdint.h>
 #include <stdio.h>
 #include <stdlib.h>
