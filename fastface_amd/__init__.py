@@ -137,6 +137,7 @@ EXPORTS = [
     ("ffk_pack_fc_weights", C.c_int, [_p, C.c_int, C.c_int, _p]),
     ("ffk_pack_fc_row", C.c_int, [_p, C.c_int, C.c_int, C.c_int, _p]),
     ("ffk_fc", C.c_int, [C.POINTER(ffk_fc_desc), _p]),
+    ("ffk_fc_variant", C.c_char_p, [C.POINTER(ffk_fc_desc)]),
     ("ffk_fc_workspace_bytes", C.c_size_t, [C.POINTER(ffk_fc_desc)]),
     ("ffk_selftest_mfma", C.c_int, []),
 ]

@@ -44,9 +44,11 @@
 namespace {
 
 // m / d by multiplication, mag = ceil(2^32 / d) (0 stands for d == 1): exact
-// for every m with m * d < 2^32, which ff_wk_geom checks for the largest m
-// of each divisor (mag * d exceeds 2^32 by less than d, so the error m *
-// (mag * d - 2^32) / (d * 2^32) stays below 1 / d)
+// for every m with m * d < 2^32 (mag * d exceeds 2^32 by less than d, so the
+// error m * (mag * d - 2^32) / (d * 2^32) stays below 1 / d).  The largest m
+// of each divisor is checked where the kernel is chosen: block indices by
+// grid_fits, pixels and K positions by the conv rules (choose_launch,
+// ffk_conv_s2_shortcut, ff_conv_generic_launch).
 __device__ __forceinline__ unsigned fdiv(unsigned m, unsigned mag) { return mag ? __umulhi(m, mag) : m; }
 
 typedef float v4f __attribute__((ext_vector_type(4)));
@@ -497,6 +499,13 @@ unsigned magic(unsigned d) { return d <= 1 ? 0u : (unsigned)((0x100000000ull + d
 struct WkTileSize { int bm, bn; };
 constexpr WkTileSize WK_TILES[WK_NTILES] = {{16, 32}, {32, 32}, {32, 64}, {48, 64}, {64, 64}};
 
+// A grid whose blocks wk_pos can divide exactly (tiles_n, then split) and
+// whose threads the launch can count.
+bool grid_fits(long long tiles, long long tiles_n, int split) {
+    const long long wgs = tiles * split, lim = 0xffffffffLL;
+    return wgs <= lim / (KW * 64) && wgs <= lim / tiles_n && wgs <= lim / split;
+}
+
 template <bool FC, typename X>
 int wk_launch(const ConvArgs& a, WkGeom& g, int tile, int split, hipStream_t s, const X& x) {
     const WkTileSize& ts = WK_TILES[tile];
@@ -609,6 +618,18 @@ WkFcPlan ff_wk_fc_plan(int batch, int n, int k, size_t ws_bytes) {
     for (int t = 0; t < WK_NTILES; t++)
         if (ff_wk_tiles(t, batch, n) <= FF_WK_MAX_WG) return {t, 1, 0};
     return {WK_NTILES - 1, 1, 0};
+}
+
+// Heads this kernel takes: buffers below 2 GiB, vectors of four outputs, and
+// a grid that fits (65537 column tiles of 64 fail from the second row tile
+// on).  A plan with fewer workgroups than FF_WK_MAX_WG always fits, so the
+// whole-K plan of the most tiles decides.
+bool ff_wk_fc_fits(int batch, int n, int k) {
+    const long long lim = 0x7fffffffLL;
+    if ((n & 3) || (long long)batch * k > lim || (long long)n * k > lim) return false;
+    const WkFcPlan p = ff_wk_fc_plan(batch, n, k, 0);
+    const int bn = WK_TILES[p.tile].bn;
+    return grid_fits(ff_wk_tiles(p.tile, batch, n), (n + bn - 1) / bn, p.split);
 }
 
 int ff_wk_fc(const ffk_fc_desc* d, hipStream_t s) {

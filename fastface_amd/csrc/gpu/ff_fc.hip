@@ -131,9 +131,7 @@ FcKernel fc_kernel(const ffk_fc_desc* d, size_t ws_bytes) {
     if (d->path == 0 && d->batch < FC_WAVEK_MIN_WHOLE && ff_wk_fc_plan(d->batch, d->n, d->k, ws_bytes).split == 1)
         return FC_MATVEC;
     if (gemm_shape && d->batch > FC_WAVEK_MAX) return FC_GEMM;
-    // its buffers hold less than 2 GiB, its vectors four outputs
-    const bool fits = (d->n & 3) == 0 && (long long)d->batch * d->k <= 0x7fffffffLL && (long long)d->n * d->k <= 0x7fffffffLL;
-    return fits ? FC_WAVEK : gemm_shape ? FC_GEMM : FC_MATVEC;
+    return ff_wk_fc_fits(d->batch, d->n, d->k) ? FC_WAVEK : gemm_shape ? FC_GEMM : FC_MATVEC;
 }
 
 }  // namespace
@@ -167,6 +165,15 @@ size_t ffk_fc_workspace_bytes(const ffk_fc_desc* d) {
     case FC_WAVEK: return ff_wk_fc_plan(d->batch, d->n, d->k, (size_t)-1).ws_bytes;
     case FC_GEMM: return ffk_fc_split_ws_bytes(d->batch);
     default: return 0;
+    }
+}
+
+const char* ffk_fc_variant(const ffk_fc_desc* d) {
+    if (!d || d->batch <= 0 || d->n <= 0 || d->k <= 0 || (d->k % FF_KSTEP) != 0) return nullptr;
+    switch (fc_kernel(d, d->workspace ? d->workspace_bytes : 0)) {
+    case FC_WAVEK: return "wavek";
+    case FC_GEMM: return d->n == 512 && d->k == 25088 ? "gemm" : nullptr;
+    default: return "matvec";
     }
 }
 

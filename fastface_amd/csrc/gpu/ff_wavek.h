@@ -26,4 +26,5 @@ int ff_wk_generic(const ConvArgs& a, const ffk_conv_desc* d, int bn, hipStream_t
 
 struct WkFcPlan { int tile, split; size_t ws_bytes; };
 WkFcPlan ff_wk_fc_plan(int batch, int n, int k, size_t ws_bytes);
+bool ff_wk_fc_fits(int batch, int n, int k);
 int ff_wk_fc(const ffk_fc_desc* d, hipStream_t s);

@@ -354,6 +354,12 @@ typedef struct {
 /* Workspace bytes ffk_fc would use for this descriptor's batch and path
  * (0: none); the workspace fields are not read. */
 size_t ffk_fc_workspace_bytes(const ffk_fc_desc* d);
+/* Name of the kernel ffk_fc would run for this descriptor's sizes, path and
+ * workspace_bytes (its pointers are not followed): "matvec", "wavek" (the
+ * MFMA kernel that shares K among the waves of a workgroup) or "gemm"
+ * (128x128 MFMA tiles); NULL when the call would be refused.  No counterpart
+ * in the reference: it lets tests name the code path they exercise. */
+const char* ffk_fc_variant(const ffk_fc_desc* d);
 size_t ffk_fc_packed_bytes(int n, int k);
 /* Packed FC weights: packed[(s*n + r)*64 + kk] = w_nk[r*k + s*64 + kk]
  * (k a multiple of 64); ffk_pack_fc_row packs row r alone (`row`: its k

@@ -129,6 +129,24 @@ def test_wavek_fc_other_heads(gpu_lib, oracle, B, K, N, split):
         assert np.array_equal(got[b], oracle.fc(a[b], W, ws, bias)), b
 
 
+@pytest.mark.parametrize("B,N,kernel", [(5, 4194368, b"matvec"), (65, 46340 * 64, b"wavek")])
+def test_fc_wide_heads(gpu_lib, oracle, B, N, kernel):
+    """Millions of outputs: the widest grid of two row tiles whose block
+    indices divide exactly, and a head past it, which the matvec runs."""
+    K = 64
+    d = fa.ffk_fc_desc()
+    d.batch, d.n, d.k = B, N, K
+    assert gpu_lib.ffk_fc_variant(C.byref(d)) == kernel
+    r = rng(3350 + B)
+    a = r.integers(-128, 128, size=(B, K), dtype=np.int8)
+    W = r.integers(-128, 128, size=(N, K), dtype=np.int8)
+    ws = r.uniform(1e-7, 1e-5, N).astype(F32)
+    bias = r.normal(0, 0.05, N).astype(F32)
+    got = run_fc(gpu_lib, a, W, ws, bias)
+    for b in sorted({0, min(B, 64) - 1, B - 1}):
+        assert np.array_equal(got[b], oracle.fc(a[b], W, ws, bias)), b
+
+
 # (cin, cout, H, shortcut's cin, batch): a stride-2 conv and its shortcut as
 # one launch, on every tile it takes, ragged last row tiles, one to four
 # shortcut steps, the first conv's steps a multiple of the waves or not

@@ -606,3 +606,28 @@ def test_fma_tail_proof_preconditions():
     assert _fma_ok(lib, 0.0, 0.0072, 1e9, 0.075, 576) == 1            # constant channel
     assert _fma_ok(lib, 0.0, 0.1515151411294937 / 1.0, float(np.float32(3.3)), 0.0, 576, prelu=False) == 0
     assert _fma_ok(lib, -1e-3, 0.1, 20.0, 0.25, 2304) == 1
+
+
+@pytest.mark.parametrize("batch,n,k", [(5, 4194368, 64), (641, 1271488, 64), (513, 1500000, 512), (577, 1500000, 512),
+                                       (200, 4000000, 64), (4097, 65536, 128), (70000, 70000, 64), (7, 500, 192),
+                                       (2048, 100000, 512), (16777216, 64, 64), (33554431, 4, 64)])
+def test_fc_grids_divide_exactly(batch, n, k):
+    """The wave-split kernel divides its block index by the column tiles with
+    a 32-bit multiplier, exact while index * divisor stays below 2^32: a head
+    whose grid goes past that takes another kernel, and on every grid it does
+    take the quotient of each row tile's first and last block is right."""
+    lib = fa.load()
+    d = fa.ffk_fc_desc()
+    d.batch, d.n, d.k = batch, n, k
+    kernel = lib.ffk_fc_variant(C.byref(d))
+    # (more tiles than CUs, but for the small head: the 64x64 tile, whole K)
+    tm, tn = -(-batch // 64), -(-n // 64)
+    mag = -(-(1 << 32) // tn) & 0xffffffff
+    quotient = lambda m: m if tn == 1 else m * mag >> 32
+    exact = all(quotient(t * tn + e) == t for t in range(tm) for e in (0, tn - 1))
+    # a workgroup of 512 threads: the launch counts them in 32 bits
+    fits = exact and tm * tn * 512 < 1 << 32
+    assert kernel in (b"wavek", b"matvec")
+    if kernel == b"wavek":
+        assert fits
+    assert (kernel == b"wavek") == (tm * tn * tn < 1 << 32 and tm * tn * 512 < 1 << 32), "the head takes the wrong kernel"
