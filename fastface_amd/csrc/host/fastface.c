@@ -502,7 +502,7 @@ static const GraphEntry* graph_for(FastFace* ff, int batch, int fmt, const Graph
  * one, 80-120 us more for a batch on an idle GPU (24 faces 695 -> 597 us, 203
  * faces 1819 -> 1617, calls with other buffers each time).  (The join is
  * made even after an error, so that nothing is left behind on the second
- * stream.) */
+ * stream; where it cannot be made the host waits for that stream.) */
 static int launch_chain(FastFace* ff, const GraphEntry* g, void* stream)
 {
     if (!g->exec2) return ffk_graph_launch(g->exec, stream);
@@ -513,6 +513,7 @@ static int launch_chain(FastFace* ff, const GraphEntry* g, void* stream)
     if (!rc) rc = ffk_graph_launch(g->exec2, ff->sstream);
     int rj = ffk_event_record(ff->ev_join, ff->sstream);
     if (!rj) rj = ffk_stream_wait_event(stream, ff->ev_join);
+    if (rj) ffk_stream_sync(ff->sstream);
     return rc ? rc : rj;
 }
 
@@ -529,8 +530,10 @@ static int enqueue_chain(FastFace* ff, int batch, void* stream, int fmt, const G
         if (!g) g = graph_for(ff, batch, fmt, NULL, NULL);
         rc = g ? launch_chain(ff, g, stream) : FFK_ERR_HIP;
     }
-    if (!rc) rc = mark_enqueued(ff, stream);
-    return rc;
+    /* (after an error too: a part of the chain may be in flight) */
+    const int rm = mark_enqueued(ff, stream);
+    if (rm) ffk_stream_sync(stream);
+    return rc ? rc : rm;
 }
 
 static int enqueue(FastFace* ff, int batch, void* stream, int fmt)
