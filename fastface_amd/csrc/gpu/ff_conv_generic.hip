@@ -794,10 +794,12 @@ int ff_conv_generic_launch(const ConvArgs& a, const ffk_conv_desc* d, hipStream_
         }
         const GenTile t = gen_tile(as.M, d->cin, d->cout);
         const dim3 gd((unsigned)grid);
-        // (its vectors hold four channels; its pixel arithmetic needs M * hout*wout below 2^32, its
-        // K arithmetic K * cin)
+        // (its vectors hold four channels and it fetches BN tables in 16-byte pieces, where the
+        // tiles here take them at any address; its pixel arithmetic needs M * hout*wout below 2^32,
+        // its K arithmetic K * cin)
+        const bool lut_ok = !(d->flags & FFK_EPI_BN) || d->out_i32 || ((uintptr_t)d->bn_lut & 15) == 0;
         if (run == 16 && t.bm == 64 && grid <= FF_WK_MAX_WG && g.kpad / FF_KSTEP >= GEN_WK_MIN_STEPS && g.vec >= 4 &&
-            as.M * px_out < 0x100000000ll && (long long)g.kpad * g.cin < 0x100000000ll) {
+            lut_ok && as.M * px_out < 0x100000000ll && (long long)g.kpad * g.cin < 0x100000000ll) {
             const int rc = ff_wk_generic(as, d, t.bn, s);
             if (rc != FFK_OK) return rc;
             continue;

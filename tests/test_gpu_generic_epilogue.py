@@ -24,7 +24,19 @@ pytestmark = pytest.mark.gpu
     (112, 128, 3, 1, 37, 11)])
 @pytest.mark.parametrize("offsets", [(0, 0, 0), (8, 8, 8), (16, 4, 0), (0, 16, 1), (3, 0, 16)])
 def test_generic_epilogue_vector_widths(gpu_lib, oracle, cin, cout, k, pad, H, B, offsets):
-    lib = gpu_lib
+    _check(gpu_lib, oracle, cin, cout, k, pad, H, B, offsets)
+
+
+# the same shapes' small grids with the BN tables at addresses that allow 8-,
+# 4- and 1-byte accesses only
+@pytest.mark.parametrize("cin,cout,k,pad,H,B", [(80, 64, 3, 1, 9, 3), (128, 36, 3, 1, 9, 2), (48, 100, 5, 2, 11, 2),
+                                                (32, 80, 3, 1, 9, 2)])
+@pytest.mark.parametrize("lut_offset", [8, 4, 1])
+def test_generic_bn_table_at_any_address(gpu_lib, oracle, cin, cout, k, pad, H, B, lut_offset):
+    _check(gpu_lib, oracle, cin, cout, k, pad, H, B, (0, 0, 0), lut_offset)
+
+
+def _check(lib, oracle, cin, cout, k, pad, H, B, offsets, lut_offset=0):
     r = rng(4100 + cin + cout * 3 + H)
     ho = H + 2 * pad - k + 1
     x = r.integers(-128, 128, size=(B, H, H, cin), dtype=np.int8)
@@ -45,11 +57,12 @@ def test_generic_epilogue_vector_widths(gpu_lib, oracle, cin, cout, k, pad, H, B
     guard = np.full(n + 64, 0x5a, np.int8)
     res = np.concatenate([np.zeros(offsets[2], np.int8), add.reshape(-1)])
     dx, dw, dp = Dev(lib, host=x), Dev(lib, host=pack_conv(lib, w)), Dev(lib, host=P)
-    dl, da = Dev(lib, host=make_bn_lut(lib, P)), Dev(lib, host=res)
+    lut = np.concatenate([np.zeros(lut_offset, np.int8), make_bn_lut(lib, P).reshape(-1)])
+    dl, da = Dev(lib, host=lut), Dev(lib, host=res)
     do, db = Dev(lib, host=guard), Dev(lib, host=guard)
     d = fa.ffk_conv_desc()
     d.batch, d.cin, d.cout, d.kh, d.kw, d.stride, d.pad, d.hin, d.win = B, cin, cout, k, k, 1, pad, H, H
-    d.in_, d.w, d.params, d.bn_lut = dx.ptr, dw.ptr, dp.ptr, dl.ptr
+    d.in_, d.w, d.params, d.bn_lut = dx.ptr, dw.ptr, dp.ptr, dl.ptr + lut_offset
     d.add_src, d.out, d.out_bn = da.ptr + offsets[2], do.ptr + offsets[0], db.ptr + offsets[1]
     d.flags = fa.FFK_EPI_BIAS | fa.FFK_EPI_PRELU | fa.FFK_EPI_ADD | fa.FFK_EPI_BN
     assert lib.ffk_conv_variant(C.byref(d)) == b"generic"
