@@ -141,6 +141,7 @@ struct FastFace {
     int n_graphs, graph_rr;
     void* ev_last;              /* recorded after the last enqueue, on last_stream */
     void* last_stream;          /* stream of the last enqueue (NULL: none pending) */
+    int last_batch, last_fmt;   /* the chain of the last enqueue */
 };
 
 static void report(const char* what, int rc)
@@ -533,11 +534,22 @@ static int enqueue_chain(FastFace* ff, int batch, void* stream, int fmt, const G
     /* (after an error too: a part of the chain may be in flight) */
     const int rm = mark_enqueued(ff, stream);
     if (rm) ffk_stream_sync(stream);
+    ff->last_batch = batch;
+    ff->last_fmt = fmt;
     return rc ? rc : rm;
 }
 
+/* The same for a whole call: a chain other than the unfinished one's is
+ * neither captured nor launched behind it, but once it has ended.  (Calls of
+ * different sizes queued without a host wait have faulted the GPU, in a build
+ * that also rewrote d_io from a kernel on the launch stream; the cause was
+ * not shown.  Equal calls queue, as one replayed graph.) */
 static int enqueue(FastFace* ff, int batch, void* stream, int fmt)
 {
+    if (ff->last_stream && (batch != ff->last_batch || fmt != ff->last_fmt)) {
+        const int rc = drain(ff);
+        if (rc) return rc;
+    }
     return enqueue_chain(ff, batch, stream, fmt, NULL);
 }
 

@@ -73,7 +73,9 @@ FastFace* fastface_create_with_scales(const char* ffw4_path, const char* opsc_pa
 int fastface_embed_batch(FastFace* ff, const float* in_bhwc, int batch, float* out_b512);
 
 /* Device-resident variant: d_in / d_out are device pointers (HBM), the work
- * is enqueued on `stream` (NULL: the context's stream) and not waited for. */
+ * is enqueued on `stream` (NULL: the context's stream) and not waited for.  A
+ * call with other buffers or another batch size than an earlier one still
+ * running waits on the host until that one has ended. */
 int fastface_embed_batch_device(FastFace* ff, const float* d_in, int batch, float* d_out,
                                 void* stream);
 

@@ -128,6 +128,9 @@ int main(int argc, char** argv)
         DEVICE(30);
         STEP("reserve");
         printf("rc %d\n", fastface_reserve(ff, MAX + 1));
+    } else if (!strcmp(sc, "sizes")) {          /* the same buffers, different batches, no wait by the caller */
+        fastface_reserve(ff, MAX);
+        DEVICE(8); DEVICE(8); DEVICE(5); DEVICE(36); DEVICE(37); DEVICE(37); DEVICE(8);
     } else {
         fprintf(stderr, "unknown scenario %s\n", sc);
         return 2;

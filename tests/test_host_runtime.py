@@ -78,3 +78,21 @@ def test_half_of_a_split_batch_fails(trace, what):
         joined = [x for x in lines[at:freed] if x.startswith("wait ") and x.split()[1] in events and not x.endswith("FAILED")
                   and x.split()[3] != s]
         assert waited or (s != streams["mine"] and joined), (s, lines)
+
+
+def test_chains_of_different_sizes_do_not_queue(trace):
+    """A device call whose batch differs from the unfinished one's waits for
+    it on the host before it launches (or captures) anything, also where the
+    buffers are the same and the I/O descriptor stays; an equal one queues."""
+    streams, calls = trace("sizes")
+    calls = [(c, lines) for c, lines in calls if c.startswith("device")]
+    assert [c for c, _ in calls] == ["device %d" % n for n in (8, 8, 5, 36, 37, 37, 8)]
+    end = None                                          # the event at the last call's end
+    for k, (c, lines) in enumerate(calls):
+        assert rc(lines) == 0
+        first = next(i for i, x in enumerate(lines) if x.startswith(("launch ", "capture ")))
+        waited = [x.split()[1] for x in lines[:first] if x.startswith("event_sync ")]
+        if k:
+            assert (end in waited) == (calls[k - 1][0] != c), (c, lines)
+        records = [x.split()[1] for x in lines if x.startswith("record ") and x.endswith("stream " + streams["mine"])]
+        end = records[-1]
