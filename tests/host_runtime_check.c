@@ -131,6 +131,11 @@ int main(int argc, char** argv)
     } else if (!strcmp(sc, "sizes")) {          /* the same buffers, different batches, no wait by the caller */
         fastface_reserve(ff, MAX);
         DEVICE(8); DEVICE(8); DEVICE(5); DEVICE(36); DEVICE(37); DEVICE(37); DEVICE(8);
+    } else if (!strcmp(sc, "host")) {           /* host batches around the pinned buffer's sizes */
+        fastface_reserve(ff, MAX);
+        HOST(1); HOST(8); HOST(2); HOST(1); HOST(8); HOST(9); HOST(1); HOST(2);
+        STEP("host 7 rgb8");
+        printf("rc %d\n", fastface_embed_batch_rgb8(ff, (const uint8_t*)in, 7, out));
     } else {
         fprintf(stderr, "unknown scenario %s\n", sc);
         return 2;

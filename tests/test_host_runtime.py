@@ -96,3 +96,16 @@ def test_chains_of_different_sizes_do_not_queue(trace):
             assert (end in waited) == (calls[k - 1][0] != c), (c, lines)
         records = [x.split()[1] for x in lines if x.startswith("record ") and x.endswith("stream " + streams["mine"])]
         end = records[-1]
+
+
+def test_small_host_outputs_go_through_pinned_memory(trace):
+    """Up to eight faces' embeddings reach the caller through the pinned
+    buffer: one fp32 face (and six uint8) in place, more by a copy into it."""
+    _, calls = trace("host")
+    for c, lines in calls:
+        if not c.startswith("host"):
+            continue
+        assert rc(lines) == 0
+        out = [x.split()[3] for x in lines if x.startswith("d2h ")]
+        n = int(c.split()[1])
+        assert out == ([] if n == 1 else ["1"] if n <= 8 else ["0"]), (c, lines)
