@@ -87,7 +87,17 @@
  * 0.640 -> 0.649, 0.694 -> 0.674, 0.766 -> 0.724, 0.727 -> 0.773). */
 #define FF_SPLIT_MIN 24
 
-/* one captured chain per (batch, input format: 0 fp32 faces, 1 uint8 RGB) */
+/* input format of a chain: 0 fp32 faces or FF_FMT_U8 uint8 RGB, over the
+ * caller's or the context's device buffers or, FF_FMT_IN_PLACE, the pinned
+ * buffer of small host batches (an I/O descriptor of its own, written once,
+ * so that calls of both kinds alternate without rewriting one: a copy
+ * between two host waits, about 20 us) */
+#define FF_FMT_U8 1
+#define FF_FMT_IN_PLACE 2
+
+#define FF_H_IO_IN_PLACE (2 * (1 + FF_MAX_CHUNKS))
+
+/* one captured chain per (batch, input format) */
 typedef struct {
     int batch, fmt;
     void* exec;                 /* the chain, or its first half */
@@ -123,9 +133,11 @@ struct FastFace {
     float* d_output;            /* capacity * 512 */
     void* d_ws;                 /* split-K workspaces of the small-batch convs */
     size_t ws_part;             /* bytes of each of d_ws's two halves */
-    ffk_io* d_io;               /* device I/O descriptors of the two halves */
+    ffk_io* d_io;               /* device I/O descriptors: [0..1] of the two
+                                   halves, [2] of the chains in place */
     ffk_io* h_io;               /* pinned staging, two descriptors each:
-                                   [0..1] set_io, [2(1 + k)..] chunk k */
+                                   [0..1] set_io, [2(1 + k)..] chunk k; then
+                                   one: FF_H_IO_IN_PLACE */
     void* cstream;              /* host-to-device copies of streamed chunks */
     void* sstream;              /* the second half of a split chain */
     void* ev_fork, *ev_join;    /* around the second half */
@@ -209,7 +221,7 @@ static int split_at(const FastFace* ff, int batch)
 }
 
 /* the I/O descriptors of the two halves of a `batch` chain over (in, out);
- * fmt 0: fp32 faces, 1: uint8 RGB */
+ * fmt 0: fp32 faces, FF_FMT_U8: uint8 RGB */
 static void io_pair(const FastFace* ff, ffk_io* io, const void* in, float* out, int batch, int fmt)
 {
     const int na = split_at(ff, batch);
@@ -332,8 +344,15 @@ static int8_t* tensor_ptr(FastFace* ff, int t, size_t off)
     return ff->d_bufs[T->buf] + off;
 }
 
+/* the device I/O descriptor of half `part` of a chain, or of one in place
+ * (never split: FF_SMALL_OUT holds eight faces) */
+static const ffk_io* io_slot(const FastFace* ff, int part, int fmt)
+{
+    return ff->d_io + ((fmt & FF_FMT_IN_PLACE) ? 2 : part);
+}
+
 /* conv descriptor of step s (pointers are NULL while no activations exist);
- * fmt 1: the input layer reads uint8 RGB pixels through the input table */
+ * FF_FMT_U8: the input layer reads uint8 RGB pixels through the input table */
 /* A conv over a tensor stored at its even pixels only (a 1x1 stride-2
  * shortcut) runs at stride 1 over the compact tensor. */
 static int reads_even(const FastFace* ff, const FfStep* st)
@@ -358,9 +377,9 @@ static void step_desc(FastFace* ff, int s, int batch, int fmt, int part, size_t 
     if (reads_even(ff, st)) { d->stride = 1; d->hin = st->hin / 2; d->win = st->win / 2; }
     if (st->t_in == FF_T_INPUT) {
         d->in = NULL;
-        d->io = ff->d_io + part;
+        d->io = io_slot(ff, part, fmt);
         d->in_inv = ff->d_in_inv;
-        if (fmt) d->in_lut = ff->d_in_lut;
+        if (fmt & FF_FMT_U8) d->in_lut = ff->d_in_lut;
     } else {
         d->in = ff->d_bufs ? tensor_ptr(ff, st->t_in, off) : NULL;
     }
@@ -372,7 +391,7 @@ static void step_desc(FastFace* ff, int s, int batch, int fmt, int part, size_t 
         d->out_bn = tensor_ptr(ff, st->t_bn, off);
     }
     if (st->flags & FFK_EPI_BN) d->bn_lut = ff->d_weights + st->lut_off;
-    d->flags = step_flags(ff, st) | ((fmt && st->t_in == FF_T_INPUT) ? FFK_IN_RGB8 : 0) |
+    d->flags = step_flags(ff, st) | (((fmt & FF_FMT_U8) && st->t_in == FF_T_INPUT) ? FFK_IN_RGB8 : 0) |
                (writes_even(ff, st) ? FFK_OUT_X_EVEN : 0);
     if (ff->algo == FASTFACE_CONV_WINOGRAD_F23 && st->wino_off != (size_t)-1) {
         d->flags |= FFK_ALGO_WINOGRAD;
@@ -410,7 +429,7 @@ static int launch_step(FastFace* ff, int s, int batch, void* stream, int fmt, in
     f.bias = ff->d_params + st->bias_off;
     f.a_scale = st->a_scale;
     f.out = NULL;
-    f.io = ff->d_io + part;
+    f.io = io_slot(ff, part, fmt);
     f.path = 0;
     f.workspace = ff->d_ws ? (int8_t*)ff->d_ws + (size_t)part * ff->ws_part : NULL;
     f.workspace_bytes = ff->ws_part;
@@ -587,8 +606,8 @@ FastFace* fastface_create_with_scales(const char* ffw4_path, const char* opsc_pa
     ff->d_params = (float*)ffk_malloc(ff->plan.p_floats * sizeof(float));
     ff->d_in_inv = (float*)ffk_malloc(4 * sizeof(float));
     ff->d_in_lut = (int8_t*)ffk_malloc(3 * 256);
-    ff->d_io = (ffk_io*)ffk_malloc(2 * sizeof(ffk_io));
-    ff->h_io = (ffk_io*)ffk_host_alloc(2 * (1 + FF_MAX_CHUNKS) * sizeof(ffk_io));
+    ff->d_io = (ffk_io*)ffk_malloc(3 * sizeof(ffk_io));
+    ff->h_io = (ffk_io*)ffk_host_alloc((FF_H_IO_IN_PLACE + 1) * sizeof(ffk_io));
     if (ffk_stream_create(&ff->cstream)) { report("stream", FFK_ERR_HIP); goto fail; }
     if (ffk_stream_create(&ff->sstream)) { report("stream", FFK_ERR_HIP); goto fail; }
     if (ffk_event_create(&ff->ev_fork) || ffk_event_create(&ff->ev_join)) { report("event", FFK_ERR_HIP); goto fail; }
@@ -666,7 +685,7 @@ int fastface_reserve(FastFace* ff, int max_batch)
 
 void* fastface_stream(FastFace* ff) { return ff ? ff->stream : NULL; }
 
-/* A batch from host memory (fmt 0: fp32 faces, 1: uint8 RGB; face_bytes
+/* A batch from host memory (fmt 0: fp32 faces, FF_FMT_U8: uint8 RGB; face_bytes
  * each) to host embeddings.  Up to one chunk: copy in, replay the chain,
  * copy out.  More: chunk k's copy goes to its own region of the input buffer
  * on the copy stream; the context stream waits for it, points the I/O
@@ -814,11 +833,22 @@ static int stage_h2d(FastFace* ff, Stager* st, int8_t* d_in, const int8_t* in, s
     return 0;
 }
 
-/* the pinned buffer of small host batches, NULL if it cannot be had (the
- * faces are then copied from and to the caller's memory) */
+/* the pinned buffer of small host batches, the descriptor of the chains in
+ * place pointed at it, or NULL if it cannot be had (the faces are then
+ * copied from and to the caller's memory) */
 static int8_t* small_buffer(FastFace* ff)
 {
-    if (!ff->h_small) ff->h_small = ffk_host_alloc_coherent(FF_SMALL_IN + FF_SMALL_OUT);
+    if (!ff->h_small) {
+        int8_t* hs = (int8_t*)ffk_host_alloc_coherent(FF_SMALL_IN + FF_SMALL_OUT);
+        if (!hs) return NULL;
+        ffk_io* slot = &ff->h_io[FF_H_IO_IN_PLACE];
+        slot->in = (const float*)hs;
+        slot->out = (float*)(hs + FF_SMALL_IN);
+        int rc = ffk_memcpy_h2d(ff->d_io + 2, slot, sizeof *slot, ff->stream);
+        if (!rc) rc = ffk_stream_sync(ff->stream);
+        if (rc) { ffk_host_free(hs); return NULL; }
+        ff->h_small = hs;
+    }
     return (int8_t*)ff->h_small;
 }
 
@@ -846,8 +876,7 @@ static int embed_host(FastFace* ff, const void* in, size_t face_bytes, int fmt, 
          * one that failed with its chain still in flight) */
         rc = ffk_stream_sync(ff->stream);
         if (!rc) memcpy(hs, in, in_bytes);
-        if (!rc) rc = set_io(ff, hs, (float*)(hs + FF_SMALL_IN), ff->stream, batch, fmt);
-        if (!rc) rc = enqueue(ff, batch, ff->stream, fmt);
+        if (!rc) rc = enqueue(ff, batch, ff->stream, fmt | FF_FMT_IN_PLACE);
     } else if (n < 2 || ff->keep_all) {
         /* one chunk: a large one still goes through the staging buffers */
         Stager* st = in_bytes >= FF_STAGE_MIN_BYTES ? staging(ff) : NULL;

@@ -109,3 +109,15 @@ def test_small_host_outputs_go_through_pinned_memory(trace):
         out = [x.split()[3] for x in lines if x.startswith("d2h ")]
         n = int(c.split()[1])
         assert out == ([] if n == 1 else ["1"] if n <= 8 else ["0"]), (c, lines)
+
+
+def test_mixed_host_batches_keep_the_descriptor(trace):
+    """Calls that run in place and calls that go through the device buffers
+    alternate without rewriting an I/O descriptor (32 bytes, a host wait
+    before and after): each kind has its own."""
+    _, calls = trace("host")
+    calls = [(c, lines) for c, lines in calls if c.startswith("host")]
+    copies = [sum(x.startswith(("h2d 16 ", "h2d 32 ")) for x in lines) for _, lines in calls]
+    # (the first call in place, the first over the device buffers, the first
+    # over the uint8 buffer)
+    assert copies == [1, 1, 0, 0, 0, 0, 0, 0, 1], list(zip([c for c, _ in calls], copies))
