@@ -16,9 +16,12 @@
 namespace {
 
 constexpr int FC_MAXB = 16;          // faces per matvec launch
-constexpr int FC_WAVEK_MIN = 3;      // the wave-split kernel's faces (fc_kernel)
-constexpr int FC_WAVEK_MIN_WHOLE = 5;
-constexpr int FC_WAVEK_MAX = 1024;
+// the wave-split kernel's faces (fc_kernel): the first with and without a K
+// split, the same for heads the matvec is quick at, and the last where the
+// 128x128 GEMM has a workspace and where it has none
+constexpr int FC_WAVEK_MIN = 3, FC_WAVEK_MIN_WHOLE = 5;
+constexpr int FC_WAVEK_MIN_QUICK = 7, FC_WAVEK_MIN_WHOLE_QUICK = 12, FC_LONG_STEPS = 512;
+constexpr int FC_WAVEK_MAX_SPLIT = 704, FC_WAVEK_MAX = 1024;
 
 __device__ __forceinline__ int dot16(v4i a, v4i w, int acc) {
     acc = __builtin_amdgcn_sdot4(a.x, w.x, acc, false);
@@ -114,23 +117,50 @@ __global__ void mfma_probe_kernel(int* out) {
     }
 }
 
-// Which kernel runs a head with ws_bytes of workspace.  The matvec's time grows with the faces (5.7 us
-// at 1, 7.3 at 2, 9.8 at 4, 27 at 16: each of its 256 workgroups reads every
-// face's activations); the wave-split kernel takes 7.7 us from 1 to 32 faces
-// and 36 at 1000, where the 128x128 tiles of the compiled GEMM take 38 (64
-// at 2000, the same); that one is compiled for the IResNet head only.
-// Without the workspace the wave-split kernel runs whole K: 10.3 us up to 24
-// faces, which passes the matvec at 5.
+// Which kernel runs a head with ws_bytes of workspace.  The matvec's time
+// grows with the faces (25088 -> 512: 5.7 us at 1, 7.0 at 2, 9.4 at 4, 26 at
+// 16: each of its workgroups reads every face's activations); the wave-split
+// kernel takes 6.8 us from 3 to 16 faces there, 28 at 512 and, without the
+// workspace (whole K), 10.3 up to 65, which passes the matvec at 5 faces.
+// Elsewhere the line lies
+// - for heads the matvec is quick at (fc_quick) at 7 faces with a split (512
+//   outputs of k = 4096: 4.2 against 5.3 us at 3 faces, 5.1 and 5.3 at 5; k =
+//   32768: 6.5 and 7.5 at 3) and at 12 without (k = 24576: 8.9 against 10.1
+//   at 8);
+// - for more than 512 K steps without a split, each wave alone with 64 of
+//   them or more, at the matvec's second launch (64 outputs of k = 98304: 32
+//   against 51 us at 16 faces);
+// - for the IResNet head at large batches, where its 128x128 GEMM's eight K
+//   ranges fill the CUs, at 704 faces with that GEMM's workspace (700: 29.9
+//   us against 31.2; 900: 34.8, 32.9; 1024: 36.8, 32.7) and at 1024
+//   without (37 against 151: its whole-K form runs 32 workgroups).
 enum FcKernel { FC_MATVEC, FC_WAVEK, FC_GEMM };
+
+// Heads the matvec is at its best for: one workgroup per CU, and a K loop of
+// one kind.  Its waves walk K in rounds of 16 steps, four rounds a pass: from
+// 49 to 63 steps per wave some lanes take a whole pass and the others a
+// remainder of three rounds, one after the other (512 outputs at 3 faces: k =
+// 24576 5.6 us, 25088 8.2, 32768 6.5).
+bool fc_quick(const ffk_fc_desc* d) {
+    const int per = (d->k / FF_KSTEP + FC_KSPLIT - 1) / FC_KSPLIT;
+    return d->n <= 256 * FC_ROWS && !(per > 48 && per < 64);
+}
 
 FcKernel fc_kernel(const ffk_fc_desc* d, size_t ws_bytes) {
     const bool gemm_shape = d->n == 512 && d->k == 25088;
-    if (d->path == 1) return FC_MATVEC;
+    if (d->path != 0 && d->path != 2) return FC_MATVEC;
     if (d->path == 2 && !gemm_shape) return FC_GEMM;               // (refused there)
-    if (d->path == 0 && d->batch < FC_WAVEK_MIN) return FC_MATVEC;
-    if (d->path == 0 && d->batch < FC_WAVEK_MIN_WHOLE && ff_wk_fc_plan(d->batch, d->n, d->k, ws_bytes).split == 1)
-        return FC_MATVEC;
-    if (gemm_shape && d->batch > FC_WAVEK_MAX) return FC_GEMM;
+    if (d->path == 0 && d->batch <= FC_MAXB) {
+        const bool split = ff_wk_fc_plan(d->batch, d->n, d->k, ws_bytes).split > 1;
+        const int least = split ? (fc_quick(d) ? FC_WAVEK_MIN_QUICK : FC_WAVEK_MIN)
+                          : d->k / FF_KSTEP > FC_LONG_STEPS ? FC_MAXB + 1
+                          : fc_quick(d) ? FC_WAVEK_MIN_WHOLE_QUICK : FC_WAVEK_MIN_WHOLE;
+        if (d->batch < least) return FC_MATVEC;
+    }
+    if (gemm_shape) {
+        const size_t gemm_ws = ffk_fc_split_ws_bytes(d->batch);
+        if (d->batch > (gemm_ws && ws_bytes >= gemm_ws ? FC_WAVEK_MAX_SPLIT : FC_WAVEK_MAX)) return FC_GEMM;
+    }
     return ff_wk_fc_fits(d->batch, d->n, d->k) ? FC_WAVEK : gemm_shape ? FC_GEMM : FC_MATVEC;
 }
 

@@ -339,9 +339,11 @@ typedef struct {
     float          a_scale;
     float*         out;      /* [batch][n] fp32, or NULL: io->out             */
     const ffk_io*  io;
-    int            path;     /* 0 auto (the matvec for 1 and 2 faces, an MFMA
-                                GEMM above), 1 matvec (16 faces per launch),
-                                2 MFMA GEMM (25088 -> 512 only)               */
+    int            path;     /* 0 auto (the matvec for a few faces and for
+                                heads whose n is not a multiple of 4, an MFMA
+                                kernel above: ffk_fc_variant), 2 an MFMA
+                                kernel (25088 -> 512 only), any other value
+                                the matvec (16 faces per launch)              */
     /* Optional workspace (device memory, zero-filled once, the same rules as
      * ffk_conv_desc.workspace; one workspace can serve both): the MFMA GEMM
      * path then shares each output tile's K reduction among several

@@ -609,7 +609,7 @@ def test_fma_tail_proof_preconditions():
 
 
 @pytest.mark.parametrize("batch,n,k", [(5, 4194368, 64), (641, 1271488, 64), (513, 1500000, 512), (577, 1500000, 512),
-                                       (200, 4000000, 64), (4097, 65536, 128), (70000, 70000, 64), (7, 500, 192),
+                                       (200, 4000000, 64), (4097, 65536, 128), (70000, 70000, 64), (33, 500, 192),
                                        (2048, 100000, 512), (16777216, 64, 64), (33554431, 4, 64)])
 def test_fc_grids_divide_exactly(batch, n, k):
     """The wave-split kernel divides its block index by the column tiles with
@@ -631,3 +631,37 @@ def test_fc_grids_divide_exactly(batch, n, k):
     if kernel == b"wavek":
         assert fits
     assert (kernel == b"wavek") == (tm * tn * tn < 1 << 32 and tm * tn * 512 < 1 << 32), "the head takes the wrong kernel"
+
+
+def _fc_variant(lib, batch, n, k, ws, path=0):
+    d = fa.ffk_fc_desc()
+    d.batch, d.n, d.k, d.path = batch, n, k, path
+    if ws:
+        d.workspace, d.workspace_bytes = 4096, lib.ffk_fc_workspace_bytes(C.byref(d))      # (not followed)
+    return (lib.ffk_fc_variant(C.byref(d)) or b"refused").decode()
+
+
+@pytest.mark.parametrize("n,k,ws,last_matvec,last_wavek", [
+    (512, 25088, True, 2, 704), (512, 25088, False, 4, 1024),          # the IResNet head, then its GEMM
+    (512, 4096, True, 6, None), (512, 4096, False, 11, None),          # one matvec workgroup per CU
+    (64, 24576, True, 6, None), (64, 24640, True, 2, None), (64, 32256, True, 2, None), (64, 32768, True, 6, None),
+    (64, 32768, False, 11, None), (64, 32832, False, 16, None), (1000, 65536, False, 16, None),
+    (516, 4096, True, 2, None), (516, 4096, False, 4, None), (100000, 512, True, 4, None),
+    (510, 25088, True, 10 ** 6, None)])                                # not a multiple of four outputs
+def test_fc_kernel_by_batch(n, k, ws, last_matvec, last_wavek):
+    """The FC kernel by the number of faces: the lines lie where the measured
+    times cross, so that no head is slower than the matvec or the GEMM it
+    would otherwise take."""
+    lib = fa.load()
+    for b in (1, 2, 3, 4, 5, 6, 7, 8, 11, 12, 16, 17, 40, 704, 705, 1024, 1025, 4000):
+        got = _fc_variant(lib, b, n, k, ws)
+        exp = "matvec" if b <= last_matvec else "gemm" if last_wavek and b > last_wavek else "wavek"
+        assert got == exp, (b, got)
+
+
+def test_fc_kernel_by_path():
+    lib = fa.load()
+    assert [_fc_variant(lib, 40, 512, 25088, True, path=p) for p in (0, 1, 2, 3)] == ["wavek", "matvec", "wavek", "matvec"]
+    assert [_fc_variant(lib, 40, 512, 4096, True, path=p) for p in (1, 2, 3)] == ["matvec", "refused", "matvec"]
+    assert _fc_variant(lib, 2, 512, 25088, True, path=2) == "wavek"
+    assert _fc_variant(lib, 0, 512, 25088, False) == _fc_variant(lib, 4, 512, 100, False) == "refused"
