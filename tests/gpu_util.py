@@ -178,7 +178,10 @@ def run_conv(lib, x, w_oihw, stride, pad, params=None, flags=0, add=None, raw=Fa
     return x_out, bn_out
 
 
-def run_fc(lib, a, W_nk, ws, bias, a_scale=1.0, path=0, split=False):
+def run_fc(lib, a, W_nk, ws, bias, a_scale=1.0, path=0, split=False, kernel=None, via_io=False):
+    """One ffk_fc call.  split: with the workspace it asks for; kernel: the
+    kernel it must run (ffk_fc_variant); via_io: the output comes through the
+    I/O descriptor, as in a captured chain."""
     a = np.ascontiguousarray(a, np.int8)
     B, K = a.shape
     N = W_nk.shape[0]
@@ -191,6 +194,9 @@ def run_fc(lib, a, W_nk, ws, bias, a_scale=1.0, path=0, split=False):
     d = fa.ffk_fc_desc()
     d.batch, d.n, d.k = B, N, K
     d.a, d.w, d.ws, d.bias, d.out = da.ptr, dw.ptr, dws.ptr, db.ptr, do.ptr
+    if via_io:
+        dio = Dev(lib, host=np.array([0, do.ptr], np.uint64))
+        d.out, d.io = None, dio.ptr
     d.a_scale = a_scale
     d.path = path
     wsp = None
@@ -200,6 +206,8 @@ def run_fc(lib, a, W_nk, ws, bias, a_scale=1.0, path=0, split=False):
         wsp = Dev(lib, nbytes=n)
         check(lib, lib.ffk_zero(wsp.ptr, n, None))
         d.workspace, d.workspace_bytes = wsp.ptr, n
+    if kernel is not None:
+        assert lib.ffk_fc_variant(C.byref(d)) == kernel
     check(lib, lib.ffk_fc(C.byref(d), None))
     check(lib, lib.ffk_stream_sync(None))
     if wsp is not None:

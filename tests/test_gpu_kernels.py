@@ -365,56 +365,53 @@ def test_config2_microbench_layer(gpu_lib, oracle):
     assert np.abs(exp.astype(np.int32)).max() == 127       # the scale reaches full range
 
 
-@pytest.mark.parametrize("B,path,split", [(1, 0, False), (3, 1, False), (16, 0, False), (17, 0, False),
-                                          (40, 2, False), (5, 2, False), (130, 0, False),
-                                          (17, 0, True), (130, 0, True), (1024, 0, True)])
-def test_fc_head(gpu_lib, oracle, B, path, split):
-    """FC head in every path: matvec (b <= 16), one MFMA GEMM workgroup per
-    128x128 output tile, and split-K (several workgroups share a tile's K
-    reduction through the workspace)."""
+@pytest.mark.parametrize("B,path,split,kernel", [
+    (1, 0, False, b"matvec"), (3, 1, False, b"matvec"), (16, 1, False, b"matvec"), (17, 1, False, b"matvec"),
+    (40, 1, False, b"matvec"), (16, 0, False, b"wavek"), (17, 0, False, b"wavek"), (40, 2, False, b"wavek"),
+    (5, 2, False, b"wavek"), (130, 0, False, b"wavek"), (17, 0, True, b"wavek"), (130, 0, True, b"wavek"),
+    (1024, 0, False, b"wavek"), (704, 0, True, b"wavek"), (705, 0, True, b"gemm"), (1024, 0, True, b"gemm"),
+    (1025, 0, False, b"gemm"), (1025, 0, True, b"gemm"), (2100, 2, False, b"gemm"), (2100, 2, True, b"gemm")])
+@pytest.mark.parametrize("via_io", [False, True])
+def test_fc_head(gpu_lib, oracle, B, path, split, kernel, via_io):
+    """FC head in every path, each named: the matvec (16 faces per launch, its
+    output rows offset per launch), the wave-split MFMA kernel, and the GEMM of
+    128x128 tiles, whole K or eight workgroups sharing a tile's K through the
+    workspace; at the batches where the choice changes, with ragged last row
+    tiles, writing to `out` or, as a captured chain does, through the I/O
+    descriptor."""
+    if via_io and B > 1025:
+        pytest.skip("the same store as at 1025 faces")
     r = rng(500 + B + path)
     K, N = 25088, 512
     a = r.integers(-128, 128, size=(B, K), dtype=np.int8)
     W = r.integers(-127, 128, size=(N, K), dtype=np.int8)
     ws = r.uniform(1e-7, 1e-5, N).astype(F32)
     bias = r.normal(0, 0.05, N).astype(F32)
-    got = run_fc(gpu_lib, a, W, ws, bias, path=path, split=split)
-    for b in (range(B) if B <= 130 else [0, 1, 127, 128, 500, B - 1]):
+    got = run_fc(gpu_lib, a, W, ws, bias, path=path, split=split, kernel=kernel, via_io=via_io)
+    for b in (range(B) if B <= 130 else [0, 1, 15, 16, 127, 128, 500, B - 2, B - 1]):
         assert np.array_equal(got[b], oracle.fc(a[b], W, ws, bias)), "face %d" % b
 
 
-@pytest.mark.parametrize("B,via_io", [(40, False), (40, True), (3, True)])
-def test_fc_other_head_shapes(gpu_lib, oracle, B, via_io):
-    """A head other than 25088 -> 512 (here K = 4096) takes the matvec at
-    every batch, 16 faces per launch, writing to `out` or, as a captured
-    chain does, through the I/O descriptor (each launch at its first face's
-    rows); the GEMM path refuses the shape."""
+@pytest.mark.parametrize("B,N,path,kernel", [(40, 512, 0, b"wavek"), (3, 512, 0, b"matvec"), (40, 512, 1, b"matvec"),
+                                             (40, 510, 0, b"matvec"), (33, 7, 0, b"matvec")])
+@pytest.mark.parametrize("via_io", [False, True])
+def test_fc_other_head_shapes(gpu_lib, oracle, B, N, path, kernel, via_io):
+    """A head other than 25088 -> 512 (here K = 4096) takes the wave-split
+    kernel or, for a few faces, where asked for, or where the outputs are no
+    multiple of four, the matvec in launches of 16 faces, each at its first
+    face's rows of `out` or of the I/O descriptor's output; the GEMM path
+    refuses the shape."""
     lib = gpu_lib
-    r = rng(570 + B)
-    K, N = 4096, 512
+    r = rng(570 + B + N)
+    K = 4096
     a = r.integers(-128, 128, size=(B, K), dtype=np.int8)
     W = r.integers(-127, 128, size=(N, K), dtype=np.int8)
     ws = r.uniform(1e-7, 1e-5, N).astype(F32)
     bias = r.normal(0, 0.05, N).astype(F32)
     exp = np.stack([oracle.fc(a[b], W, ws, bias) for b in range(B)])
-    if not via_io:
-        assert np.array_equal(run_fc(lib, a, W, ws, bias), exp)
-        with pytest.raises(RuntimeError):
-            run_fc(lib, a, W, ws, bias, path=2)
-        return
-    packed = np.empty(lib.ffk_fc_packed_bytes(N, K), np.int8)
-    gpu_util.check(lib, lib.ffk_pack_fc_weights(W.ctypes.data, N, K, packed.ctypes.data))
-    da, dw = gpu_util.Dev(lib, host=a), gpu_util.Dev(lib, host=packed)
-    dws, db = gpu_util.Dev(lib, host=ws), gpu_util.Dev(lib, host=bias)
-    do = gpu_util.Dev(lib, nbytes=B * N * 4)
-    dio = gpu_util.Dev(lib, host=np.array([0, do.ptr], np.uint64))
-    d = fa.ffk_fc_desc()
-    d.batch, d.n, d.k = B, N, K
-    d.a, d.w, d.ws, d.bias, d.out, d.io = da.ptr, dw.ptr, dws.ptr, db.ptr, None, dio.ptr
-    d.a_scale = 1.0
-    gpu_util.check(lib, lib.ffk_fc(C.byref(d), None))
-    gpu_util.check(lib, lib.ffk_stream_sync(None))
-    assert np.array_equal(do.get(np.float32, (B, N)), exp)
+    assert np.array_equal(run_fc(lib, a, W, ws, bias, path=path, kernel=kernel, via_io=via_io), exp)
+    with pytest.raises(RuntimeError):
+        run_fc(lib, a, W, ws, bias, path=2, via_io=via_io)
 
 
 @pytest.mark.parametrize("B", [1, 2, 16])

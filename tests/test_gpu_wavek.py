@@ -1,4 +1,4 @@
-"""The wave-split kernel (FFK_LATENCY convs, the FC head of 3 to 1024 faces)
+"""The wave-split kernel (FFK_LATENCY convs, the FC head from a few faces on)
 at the edges of its tiles and of its launch rules, bit for bit against the
 oracle."""
 import ctypes as C
@@ -99,8 +99,9 @@ def _check_conv(lib, oracle, cin, cout, k, s, H, B, grid, mode, L, kind):
 
 
 # batches at the ends of every tile and K split of the rule, with the
-# workspace the call asks for and without one (whole K)
-@pytest.mark.parametrize("B", [3, 4, 5, 16, 17, 64, 65, 128, 129, 256, 257, 512, 513, 1024])
+# workspace the call asks for and without one (whole K, from 5 faces); past
+# 704 faces the call's own workspace is the 128x128 GEMM's
+@pytest.mark.parametrize("B", [3, 4, 5, 16, 17, 64, 65, 128, 129, 256, 257, 512, 513, 704, 1024])
 @pytest.mark.parametrize("split", [True, False])
 def test_wavek_fc(gpu_lib, oracle, B, split):
     r = rng(3200 + B)
@@ -111,12 +112,14 @@ def test_wavek_fc(gpu_lib, oracle, B, split):
     W[-1] = -127
     ws = r.uniform(1e-7, 1e-5, N).astype(F32)
     bias = r.normal(0, 0.05, N).astype(F32)
-    got = run_fc(gpu_lib, a, W, ws, bias, a_scale=0.37, split=split)
+    kernel = (b"gemm" if B > 704 else b"wavek") if split else b"matvec" if B < 5 else b"wavek"
+    got = run_fc(gpu_lib, a, W, ws, bias, a_scale=0.37, split=split, kernel=kernel)
     for b in sorted({0, B // 2, B - 1}):
         assert np.array_equal(got[b], oracle.fc(a[b], W, ws, bias, 0.37)), b
 
 
-@pytest.mark.parametrize("B,K,N,split", [(3, 64, 12, False), (7, 192, 500, True), (33, 4096, 512, True), (70, 1024, 40, True)])
+@pytest.mark.parametrize("B,K,N,split", [(12, 64, 12, False), (7, 192, 500, True), (33, 4096, 512, True), (70, 1024, 40, True),
+                                         (3, 64, 600, True), (3, 24640, 20, True), (17, 33024, 64, False), (9, 128, 20000, False)])
 def test_wavek_fc_other_heads(gpu_lib, oracle, B, K, N, split):
     """Heads of other sizes: fewer K steps than waves, columns past N."""
     r = rng(3300 + B)
@@ -124,7 +127,7 @@ def test_wavek_fc_other_heads(gpu_lib, oracle, B, K, N, split):
     W = r.integers(-128, 128, size=(N, K), dtype=np.int8)
     ws = r.uniform(1e-7, 1e-5, N).astype(F32)
     bias = r.normal(0, 0.05, N).astype(F32)
-    got = run_fc(gpu_lib, a, W, ws, bias, split=split)
+    got = run_fc(gpu_lib, a, W, ws, bias, split=split, kernel=b"wavek")
     for b in range(B):
         assert np.array_equal(got[b], oracle.fc(a[b], W, ws, bias)), b
 
