@@ -51,7 +51,10 @@ namespace {
 // ffk_conv_s2_shortcut, ff_conv_generic_launch).
 __device__ __forceinline__ unsigned fdiv(unsigned m, unsigned mag) { return mag ? __umulhi(m, mag) : m; }
 
+// four floats or sums in the caller's memory, which is aligned to one
 typedef float v4f __attribute__((ext_vector_type(4)));
+typedef float v4f_mem __attribute__((ext_vector_type(4), aligned(4)));
+typedef int v4i_mem __attribute__((ext_vector_type(4), aligned(4)));
 
 constexpr int KW = 8;                                       // waves per workgroup
 
@@ -155,16 +158,16 @@ __device__ __forceinline__ void wk_prefetch(const ConvArgs& a, const WkGeom& g, 
     e.ws = e.bias = e.slope = e.adds = e.inv = v4f{0, 0, 0, 0};
     if constexpr (FC) {
         if (nc < g.cout) {
-            e.ws = *reinterpret_cast<const v4f*>(a.fc_ws + nc);
-            e.bias = *reinterpret_cast<const v4f*>(a.fc_bias + nc);
+            e.ws = *reinterpret_cast<const v4f_mem*>(a.fc_ws + nc);
+            e.bias = *reinterpret_cast<const v4f_mem*>(a.fc_bias + nc);
         }
     } else if (!a.out_i32 && nc < g.cout) {
         const float* P = a.params + nc;
-        e.ws = *reinterpret_cast<const v4f*>(P + FFK_P_WS * g.cout);
-        e.bias = *reinterpret_cast<const v4f*>(P + FFK_P_BIAS * g.cout);
-        e.inv = *reinterpret_cast<const v4f*>(P + FFK_P_INV * g.cout);
-        if (a.flags & FFK_EPI_PRELU) e.slope = *reinterpret_cast<const v4f*>(P + FFK_P_SLOPE * g.cout);
-        if (a.flags & FFK_EPI_ADD) e.adds = *reinterpret_cast<const v4f*>(P + FFK_P_ADDSCALE * g.cout);
+        e.ws = *reinterpret_cast<const v4f_mem*>(P + FFK_P_WS * g.cout);
+        e.bias = *reinterpret_cast<const v4f_mem*>(P + FFK_P_BIAS * g.cout);
+        e.inv = *reinterpret_cast<const v4f_mem*>(P + FFK_P_INV * g.cout);
+        if (a.flags & FFK_EPI_PRELU) e.slope = *reinterpret_cast<const v4f_mem*>(P + FFK_P_SLOPE * g.cout);
+        if (a.flags & FFK_EPI_ADD) e.adds = *reinterpret_cast<const v4f_mem*>(P + FFK_P_ADDSCALE * g.cout);
         if ((a.flags & FFK_EPI_ADD) && !PAIR) {            // (a pair's residual is its own first result)
             const __amdgpu_buffer_rsrc_t r_add = ff_rsrc(a.add_src, (unsigned)a.M * g.cout);
 #pragma unroll
@@ -234,9 +237,9 @@ __device__ __forceinline__ void wk_finish(const v4i (&acc)[MT][NT], const ConvAr
         // the first conv's int8 results, then the shortcut's sums
         v4f ws = {}, bias = {}, inv = {};
         if (nok) {
-            ws = *reinterpret_cast<const v4f*>(first.params + FFK_P_WS * g.cout + nc);
-            bias = *reinterpret_cast<const v4f*>(first.params + FFK_P_BIAS * g.cout + nc);
-            inv = *reinterpret_cast<const v4f*>(first.params + FFK_P_INV * g.cout + nc);
+            ws = *reinterpret_cast<const v4f_mem*>(first.params + FFK_P_WS * g.cout + nc);
+            bias = *reinterpret_cast<const v4f_mem*>(first.params + FFK_P_BIAS * g.cout + nc);
+            inv = *reinterpret_cast<const v4f_mem*>(first.params + FFK_P_INV * g.cout + nc);
         }
         __syncthreads();                                     // the first partial tiles are read
         int32_t* ps = reinterpret_cast<int32_t*>(smem);
@@ -309,7 +312,7 @@ __device__ __forceinline__ void wk_finish(const v4i (&acc)[MT][NT], const ConvAr
                 v4f o;
 #pragma unroll
                 for (int e = 0; e < 4; e++) o[e] = ff::fc_out(sum[q][e], a.in_scale, ep.ws[e], ep.bias[e]);
-                *reinterpret_cast<v4f*>(out + (size_t)m * g.cout + nc) = o;
+                *reinterpret_cast<v4f_mem*>(out + (size_t)m * g.cout + nc) = o;
             }
         }
         return;
@@ -325,7 +328,7 @@ __device__ __forceinline__ void wk_finish(const v4i (&acc)[MT][NT], const ConvAr
         const int m = p.m0 + gi / C4;
         if (m >= a.M || !nok) continue;
         if (a.out_i32) {
-            *reinterpret_cast<v4i*>(a.out_i32 + (size_t)m * g.cout + nc) = sum[q];
+            *reinterpret_cast<v4i_mem*>(a.out_i32 + (size_t)m * g.cout + nc) = sum[q];
             continue;
         }
         uint32_t x = 0, bn = 0;

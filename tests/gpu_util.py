@@ -178,10 +178,12 @@ def run_conv(lib, x, w_oihw, stride, pad, params=None, flags=0, add=None, raw=Fa
     return x_out, bn_out
 
 
-def run_fc(lib, a, W_nk, ws, bias, a_scale=1.0, path=0, split=False, kernel=None, via_io=False):
+def run_fc(lib, a, W_nk, ws, bias, a_scale=1.0, path=0, split=False, kernel=None, via_io=False,
+           skew=0):
     """One ffk_fc call.  split: with the workspace it asks for; kernel: the
     kernel it must run (ffk_fc_variant); via_io: the output comes through the
-    I/O descriptor, as in a captured chain."""
+    I/O descriptor, as in a captured chain; skew: scales, biases and outputs
+    start that many floats past a 16-byte address."""
     a = np.ascontiguousarray(a, np.int8)
     B, K = a.shape
     N = W_nk.shape[0]
@@ -189,13 +191,15 @@ def run_fc(lib, a, W_nk, ws, bias, a_scale=1.0, path=0, split=False, kernel=None
     check(lib, lib.ffk_pack_fc_weights(np.ascontiguousarray(W_nk, np.int8).ctypes.data, N, K,
                                        packed.ctypes.data))
     da, dw = Dev(lib, host=a), Dev(lib, host=packed)
-    dws, db = Dev(lib, host=np.asarray(ws, np.float32)), Dev(lib, host=np.asarray(bias, np.float32))
-    do = Dev(lib, nbytes=B * N * 4)
+    pad = np.zeros(skew, np.float32)
+    dws, db = (Dev(lib, host=np.concatenate([pad, np.asarray(v, np.float32)])) for v in (ws, bias))
+    do = Dev(lib, nbytes=(skew + B * N) * 4)
+    outp = do.ptr + skew * 4
     d = fa.ffk_fc_desc()
     d.batch, d.n, d.k = B, N, K
-    d.a, d.w, d.ws, d.bias, d.out = da.ptr, dw.ptr, dws.ptr, db.ptr, do.ptr
+    d.a, d.w, d.ws, d.bias, d.out = da.ptr, dw.ptr, dws.ptr + skew * 4, db.ptr + skew * 4, outp
     if via_io:
-        dio = Dev(lib, host=np.array([0, do.ptr], np.uint64))
+        dio = Dev(lib, host=np.array([0, outp], np.uint64))
         d.out, d.io = None, dio.ptr
     d.a_scale = a_scale
     d.path = path
@@ -212,4 +216,4 @@ def run_fc(lib, a, W_nk, ws, bias, a_scale=1.0, path=0, split=False, kernel=None
     check(lib, lib.ffk_stream_sync(None))
     if wsp is not None:
         assert split_counters_zero(lib, wsp)
-    return do.get(np.float32, (B, N))
+    return do.get(np.float32, (skew + B * N,))[skew:].reshape(B, N)

@@ -132,6 +132,20 @@ def test_wavek_fc_other_heads(gpu_lib, oracle, B, K, N, split):
         assert np.array_equal(got[b], oracle.fc(a[b], W, ws, bias)), b
 
 
+@pytest.mark.parametrize("via_io", [False, True])
+@pytest.mark.parametrize("skew", [1, 2, 3])
+def test_wavek_fc_at_any_float(gpu_lib, oracle, skew, via_io):
+    """Scales, biases and outputs at addresses aligned to one float only."""
+    r = rng(3320 + skew)
+    B, K, N = 40, 1024, 72
+    a = r.integers(-128, 128, size=(B, K), dtype=np.int8)
+    W = r.integers(-128, 128, size=(N, K), dtype=np.int8)
+    ws = r.uniform(1e-7, 1e-5, N).astype(F32)
+    bias = r.normal(0, 0.05, N).astype(F32)
+    got = run_fc(gpu_lib, a, W, ws, bias, kernel=b"wavek", via_io=via_io, skew=skew)
+    assert np.array_equal(got, np.stack([oracle.fc(a[b], W, ws, bias) for b in range(B)]))
+
+
 @pytest.mark.parametrize("B,N,kernel", [(5, 4194368, b"matvec"), (65, 46340 * 64, b"wavek")])
 def test_fc_wide_heads(gpu_lib, oracle, B, N, kernel):
     """Millions of outputs: the widest grid of two row tiles whose block
