@@ -22,13 +22,13 @@
  * and, one line per region, "conv|wino|bn|map|add|fc <op> <offset> <bytes>" to
  * <dump>.txt, and the parameter arena to <dump>.params.bin.  With
  * --launches, the launch list of the chain at each batch, one line per
- * launch ("launch <batch>[/h<half>] <step> conv|fc <variant> <workgroups>
- * <geometry> <flags>", or "... map|add <channels> <pixels>" for a
- * stand-alone BN / PReLU / Add), built as fastface.c builds its descriptors (two
- * halves from 24 faces, FFK_SHARED_GPU) from the library's host-side
- * launch choice: no device is involved.  The convs are listed as a caller
- * without the chain's FFK_LATENCY hint gets them; an fc line names the
- * batch's size class (up to 16 faces "matvec"). */
+ * launch ("launch <batch>[/h<half>] <step> conv <variant> <workgroups>
+ * <geometry> <flags>", "... fc <variant> <workspace bytes>" or "...
+ * map|add <channels> <pixels>" for a stand-alone BN / PReLU / Add), built as
+ * fastface.c builds its descriptors (FFK_LATENCY; two halves from 24 faces,
+ * FFK_SHARED_GPU) from the library's host-side launch choice: no device is
+ * involved.  A stride-2 conv and its shortcut are two lines also where
+ * ffk_conv_s2_shortcut would run them as one launch. */
 #include <stdint.h>
 #include <stdio.h>
 #include <stdlib.h>
@@ -47,7 +47,10 @@ static void print_launches(const FfPlan* p, const char* tag, int batch, int shar
             ffk_fc_desc f;
             memset(&f, 0, sizeof f);
             f.batch = batch; f.n = st->fc_n; f.k = st->fc_k;
-            printf("launch %s %d fc %s %zu\n", tag, s, batch <= 16 ? "matvec" : "gemm", ffk_fc_workspace_bytes(&f));
+            f.workspace = (void*)(uintptr_t)4096;        /* (never dereferenced) */
+            f.workspace_bytes = (size_t)1 << 30;
+            const char* v = ffk_fc_variant(&f);
+            printf("launch %s %d fc %s %zu\n", tag, s, v ? v : "none", ffk_fc_workspace_bytes(&f));
             continue;
         }
         if (st->kind == FF_STEP_MAP || st->kind == FF_STEP_ADD) {
@@ -63,7 +66,7 @@ static void print_launches(const FfPlan* p, const char* tag, int batch, int shar
             d.stride = 1; d.hin = st->hin / 2; d.win = st->win / 2;
         }
         d.flags = st->flags | ((st->t_out >= 0 && p->tensors[st->t_out].even) ? FFK_OUT_X_EVEN : 0) |
-                  (shared ? FFK_SHARED_GPU : 0);
+                  FFK_LATENCY | (shared ? FFK_SHARED_GPU : 0);
         d.workspace = (void*)(uintptr_t)4096;            /* (never dereferenced) */
         d.workspace_bytes = (size_t)1 << 30;
         const char* v = ffk_conv_variant(&d);

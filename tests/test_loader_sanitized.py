@@ -261,7 +261,9 @@ def test_launch_lists_without_a_gpu(checker, synth_ffw4):
     24), from the plan and the library's host-side launch choice: 53 convs +
     the FC per chain or half, every conv with a kernel variant and (but the
     persistent input layer) a workgroup count; small batches take the
-    split-K / small-grid variants, 512-face halves the large tiles."""
+    wave-split and small patch tiles of the chain's FFK_LATENCY launches, not
+    the ones of a single launch, 512-face halves the large tiles; the FC by
+    its own rule."""
     env = dict(os.environ, ASAN_OPTIONS="detect_leaks=1:abort_on_error=0")
     r = subprocess.run([checker, synth_ffw4, synth.OPSC_PATH, synth.OPSC2_PATH, "-", "--launches",
                         "1", "8", "256", "1024"], capture_output=True, text=True, env=env, timeout=120)
@@ -276,12 +278,14 @@ def test_launch_lists_without_a_gpu(checker, synth_ffw4):
         assert len(launches) == 54, tag
         for t in launches:
             if t[3] == "fc":
-                assert t[4] == ("matvec" if tag in ("1", "8") else "gemm"), t
+                assert t[4] == ("matvec" if tag == "1" else "wavek"), t
                 continue
             assert t[4] != "none", t
             assert int(t[5]) > 0 or t[4] == "stem", t
     variants = lambda tag: {t[4] for t in chains[tag]}
-    assert "splitk" in variants("1") and "splitk" not in variants("1024/h0")
+    assert not any("splitk" in variants(tag) for tag in chains)
+    assert sum(t[4] == "wavek" for t in chains["1"]) == 50 and {"wavek", "patch_kg"} <= variants("8")
+    assert "tile64" not in variants("1024/h0")
     assert "patch_kg" not in variants("1024/h0") and "patch" in variants("1024/h0")
 
 
