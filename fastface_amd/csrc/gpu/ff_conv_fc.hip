@@ -1,5 +1,5 @@
-// ff_conv_fc.hip -- the FC head 25088 -> 512 as an MFMA GEMM (batches over
-// 1024 faces): conv_i8_kernel run as a 1x1 "conv" over a 1x1 image with
+// ff_conv_fc.hip -- the FC head 25088 -> 512 as an MFMA GEMM (large batches,
+// fc_kernel in ff_fc.hip): conv_i8_kernel run as a 1x1 "conv" over a 1x1 image with
 // Cin = K, optionally with split-K through the conv workspace.
 #include "ff_conv_table.h"
 

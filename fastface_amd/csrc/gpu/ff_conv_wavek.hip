@@ -30,11 +30,11 @@
 // the launch rule stops.
 //
 // The FC head (K = 25088, 392 steps) also splits K over workgroups, four
-// ways where that fits the CUs, through the split-K workspace: 13 faces
-// 22.7 -> 7.1 us against the matvec, 100 faces 29.1 -> 10.1 and 512 faces
-// 31.4 -> 22.4 against 128x128 tiles split eight ways (32 to 128
-// workgroups).  Two faces are equal to the matvec (7.3), one is slower
-// (5.7 there).
+// ways where that fits the CUs, through the split-K workspace: 12 faces
+// 20.4 -> 6.9 us against the matvec, 100 faces 28.5 -> 9.6 and 512 faces
+// 30.3 -> 22.7 against 128x128 tiles split eight ways (32 to 128
+// workgroups).  Where the matvec and, past 704 faces, those tiles are the
+// faster ones: fc_kernel.
 #include "ff_conv_table.h"
 #include "ff_numerics.h"
 #include "ff_wavek.h"
@@ -605,7 +605,7 @@ int ff_wk_generic(const ConvArgs& a, const ffk_conv_desc* d, int bn, hipStream_t
 }
 
 // The FC head: four K ranges where a tile's grid then fits the CUs, two with
-// the 64x64 tiles above that (513-1024 faces of 512 outputs), else one.
+// the 64x64 tiles above that (513 to 1024 faces of 512 outputs), else one.
 // (Measured with 1, 2, 4, 7, 8, 14, 16 and 28 ranges at 1-2000 faces: four is
 // the fastest up to 512; more ranges pay more for the exchange than their
 // shorter loops save.)  ws_bytes: the workspace at hand; a plan that needs

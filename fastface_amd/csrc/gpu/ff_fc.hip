@@ -7,8 +7,8 @@
 // 16 B per lane per load, v_dot4 signed int8 products into exact int32), so
 // that the whole 12.8 MB weight matrix is in flight at once; the batch's
 // activation rows come from L2.  Cross-lane and then cross-wave (LDS) sums
-// give the exact dot product per face.  From three faces on the MFMA kernels
-// run it as a 1x1 conv (ff_conv_wavek.hip, ff_conv_fc.hip above 1024 faces).
+// give the exact dot product per face.  From a few faces on the MFMA kernels
+// run it as a 1x1 conv (ff_conv_wavek.hip, then ff_conv_fc.hip: fc_kernel).
 #include <cstring>
 #include "ff_numerics.h"
 #include "ff_wavek.h"

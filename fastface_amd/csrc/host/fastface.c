@@ -80,11 +80,13 @@
  * 256 2.75 -> 2.33, 512 4.37 -> 3.76, 1024 7.86 -> 7.25; with the small-tile
  * kernels of small grids the halves win from 24 faces on: 16 0.516 -> 0.586,
  * 20 0.519 -> 0.566, 24 0.625 -> 0.588, 32 0.643 -> 0.637, 40 0.728 -> 0.684,
- * 47 0.872 -> 0.722.  With the small patch tiles of FFK_LATENCY launches the
- * two are about equal up to 40 faces (24 0.569 -> 0.565, 28 0.598 -> 0.573,
- * 37 0.660 -> 0.619, 40 0.621 -> 0.672; with changing buffers 0.589 -> 0.622,
- * 0.618 -> 0.631, 0.681 -> 0.676, 0.641 -> 0.728; uint8 faces from the host
- * 0.640 -> 0.649, 0.694 -> 0.674, 0.766 -> 0.724, 0.727 -> 0.773). */
+ * 47 0.872 -> 0.722.  With the small patch tiles of FFK_LATENCY launches
+ * neither form wins throughout from 24 to 40 faces (24 0.569 -> 0.565, 28
+ * 0.598 -> 0.573, 37 0.660 -> 0.619, 40 0.621 -> 0.672; with changing buffers
+ * 0.589 -> 0.622, 0.618 -> 0.631, 0.681 -> 0.676, 0.641 -> 0.728; uint8 faces
+ * from the host 0.640 -> 0.649, 0.694 -> 0.674, 0.766 -> 0.724, 0.727 ->
+ * 0.773): it goes by how the grids fill the CUs, and another constant only
+ * moves the loss.  24 is kept. */
 #define FF_SPLIT_MIN 24
 
 /* input format of a chain: 0 fp32 faces or FF_FMT_U8 uint8 RGB, over the

@@ -355,6 +355,7 @@ def time_fc(lib, batch=1, iters=50, path=0):
     if n_ws:
         d.workspace, d.workspace_bytes = dev(nbytes=n_ws), n_ws
         assert lib.ffk_zero(d.workspace, n_ws, None) == 0, fa.last_error()
+    kernel = (lib.ffk_fc_variant(C.byref(d)) or b"").decode()
     stream, e0, e1, ms = C.c_void_p(), C.c_void_p(), C.c_void_p(), C.c_float()
     lib.ffk_stream_create(C.byref(stream))
     lib.ffk_event_create(C.byref(e0))
@@ -376,7 +377,7 @@ def time_fc(lib, batch=1, iters=50, path=0):
             lib.ffk_free(p)
     per = ms.value / iters
     return {"layer": "fc 25088->512", "batch": batch, "split_ws_bytes": n_ws,
-            "path": {1: "matvec", 2: "gemm"}.get(path, "matvec" if batch <= 16 else "gemm"),
+            "path": kernel,
             "ms_per_launch": round(per, 5),
             "weight_gbs": round(N * K / (per * 1e-3) / 1e9, 1),
             "int8_tops": round(2.0 * batch * N * K / (per * 1e-3) / 1e12, 2)}
