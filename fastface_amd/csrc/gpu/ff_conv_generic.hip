@@ -592,8 +592,14 @@ __global__ __launch_bounds__(256, 4) void conv_generic_dma_kernel(ConvArgs a, Ge
     constexpr int LPS = A_LD + B_LD;                   // loads per thread and stage
     static_assert((GEN_NST - 2) * LPS < 64, "vmcnt range");
     constexpr int LDS_K = GEN_NST * STAGE, LDS_E = gen_epi_bytes(BM, BN, LUT);
-    __shared__ __align__(1024) int8_t smem[LDS_K > LDS_E ? LDS_K : LDS_E];
-    __shared__ __align__(16) float prm[GEN_NPRM * BN];
+    // (one array for all of it: beside a second one the compiler waits for every
+    // load into LDS before it reads LDS, so that no load overlaps the step
+    // before it: 512->33 7x7 s2 @5 at 2 faces 124 us, 101 with one; 320->33 7x7
+    // @35 at 21 faces 117, 101; 5x5 256->256 @14 at 256 faces, four workgroups
+    // per CU, the same)
+    constexpr int LDS = LDS_K > LDS_E ? LDS_K : LDS_E;
+    __shared__ __align__(1024) int8_t smem[LDS + GEN_NPRM * BN * 4];
+    float* prm = reinterpret_cast<float*>(smem + LDS);
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lane = tid & 63;

@@ -665,3 +665,21 @@ def test_fc_kernel_by_path():
     assert [_fc_variant(lib, 40, 512, 4096, True, path=p) for p in (1, 2, 3)] == ["matvec", "refused", "matvec"]
     assert _fc_variant(lib, 2, 512, 25088, True, path=2) == "wavek"
     assert _fc_variant(lib, 0, 512, 25088, False) == _fc_variant(lib, 4, 512, 100, False) == "refused"
+
+
+def test_kernels_with_lds_loads_declare_one_lds_array():
+    """A kernel that loads straight into LDS keeps all of its LDS in one
+    array: with a second one the compiler marks the two as not aliasing and,
+    tracking the loads from then on, waits for all of them before every LDS
+    read, so that no load overlaps the K step before it."""
+    gpu = os.path.join(fa.REPO_ROOT, "fastface_amd", "csrc", "gpu")
+    seen = 0
+    for name in sorted(os.listdir(gpu)):
+        src = re.sub(r"//[^\n]*|/\*.*?\*/", "", open(os.path.join(gpu, name)).read(), flags=re.S)
+        for kernel in src.split("__global__")[1:]:
+            body = kernel[:kernel.find("\n}\n")]
+            if not re.search(r"\bb?dma16\(", body):
+                continue
+            seen += 1
+            assert body.count("__shared__") == 1, (name, body[:200])
+    assert seen >= 5
