@@ -636,21 +636,39 @@ __global__ __launch_bounds__(256, 4) void conv_generic_dma_kernel(ConvArgs a, Ge
         const int n = n0 + ((j * 4 + wave) * 4 + (lane >> 4)) * 4 + (sl >> 2);
         b_off[j] = n < g.cout ? (unsigned)(n * 64 + p * 16) : FF_OOB;
     }
+    // A step's A offsets.  64-row tiles are taken where there is about one
+    // workgroup per CU and nothing else hides the chain of their arithmetic: they
+    // are computed a step ahead, in the shadow of the fragment reads (512->33
+    // 7x7 s2 @5 at 2 faces 101 -> 91 us, 320->33 7x7 @35 at 21 faces 101 ->
+    // 90).  128-row tiles compute them at the loads: other workgroups of the
+    // CU run meanwhile, and two more live registers cost more (5x5 256->256 @14
+    // at 256 faces 102 us, 107 a step ahead).
+    constexpr bool AHEAD = BM == 64;
     KCursor cur = kcursor_at(g, p * 16);
+    auto a_offset = [&](int j) {
+        const bool v = cur.k < g.ktot && (unsigned)(a_ih0[j] + cur.th) < (unsigned)g.hin &&
+                       (unsigned)(a_iw0[j] + cur.tw) < (unsigned)g.win;
+        return v ? (unsigned)(a_base[j] + cur.off) : FF_OOB;
+    };
+    unsigned a_off[A_LD] = {};
+    auto ahead = [&]() {
+        if constexpr (AHEAD) {
+#pragma unroll
+            for (int j = 0; j < A_LD; j++) a_off[j] = a_offset(j);
+            kcursor_next(cur, g);
+        }
+    };
+    ahead();
     auto issue = [&](int st, int buf) {
         int8_t* sb = smem + buf * STAGE;
-        const bool kin = cur.k < g.ktot;
 #pragma unroll
-        for (int j = 0; j < A_LD; j++) {
-            const bool v = kin && (unsigned)(a_ih0[j] + cur.th) < (unsigned)g.hin &&
-                           (unsigned)(a_iw0[j] + cur.tw) < (unsigned)g.win;
-            bdma16(r_in, v ? (unsigned)(a_base[j] + cur.off) : FF_OOB, 0u, sb + (j * 4 + wave) * 1024);
-        }
+        for (int j = 0; j < A_LD; j++)
+            bdma16(r_in, AHEAD ? a_off[j] : a_offset(j), 0u, sb + (j * 4 + wave) * 1024);
         const unsigned wst = (unsigned)(st * g.cout * 64);
 #pragma unroll
         for (int j = 0; j < B_LD; j++)
             bdma16(r_w, b_off[j], wst, sb + A_BYTES + (j * 4 + wave) * 1024);
-        kcursor_next(cur, g);
+        if constexpr (!AHEAD) kcursor_next(cur, g);
     };
 
     const int wm = wave >> 1, wn = wave & 1;
@@ -664,8 +682,10 @@ __global__ __launch_bounds__(256, 4) void conv_generic_dma_kernel(ConvArgs a, Ge
 #pragma unroll
             for (int e = 0; e < 16; e++) acc[i][j][e] = 0;
 #pragma unroll
-    for (int u = 0; u < GEN_NST - 1; u++)
+    for (int u = 0; u < GEN_NST - 1; u++) {
         if (u < nsteps) issue(u, u);
+        ahead();
+    }
     gen_params<BN>(a, g, n0, prm);
     int rbuf = 0;                                      // ring slot of step s
     for (int st = 0; st < nsteps; st++) {
@@ -680,6 +700,7 @@ __global__ __launch_bounds__(256, 4) void conv_generic_dma_kernel(ConvArgs a, Ge
             for (int i = 0; i < MI; i++) af[i] = *reinterpret_cast<const v4i*>(sb + ((a_rd + i * 2048) ^ (ks * 32)));
 #pragma unroll
             for (int j = 0; j < NJ; j++) bf[j] = *reinterpret_cast<const v4i*>(sb + ((b_rd + j * 2048) ^ (ks * 32)));
+            if (ks == 0) ahead();
 #pragma unroll
             for (int i = 0; i < MI; i++)
 #pragma unroll
