@@ -167,8 +167,9 @@ __device__ __forceinline__ v4i gather_a(const ConvArgs& a, const GenGeom& g, __a
 // @45 PReLU at 33 faces 27.4 us, now 17.0; 96->128 @35 residual+BN at 196 faces
 // 129 us, now 60.)
 
-// Channels per vector of the int8 tensors' accesses: 16, 8, 4 or 1 bytes, the
-// largest that divides the channel count and every base address.
+// Channels per vector of the int8 tensors' accesses: 16, 8 or 4 bytes, the
+// largest that divides the channel count and every base address; else 1
+// (row_bytes).
 __device__ __forceinline__ v4i chunk_load(const int8_t* p, int left, int vec) {
     v4i v = {0, 0, 0, 0};
     if (vec == 16) {
@@ -186,15 +187,9 @@ __device__ __forceinline__ v4i chunk_load(const int8_t* p, int left, int vec) {
             }
         return v;
     }
-    if (vec == 4) {
 #pragma unroll
-        for (int h = 0; h < 4; h++)
-            if (left >= 4 * h + 4) v[h] = *reinterpret_cast<const int*>(p + 4 * h);
-        return v;
-    }
-#pragma unroll
-    for (int e = 0; e < 16; e++)
-        if (e < left) v[e >> 2] |= (int)((uint32_t)(uint8_t)p[e] << (8 * (e & 3)));
+    for (int h = 0; h < 4; h++)
+        if (left >= 4 * h + 4) v[h] = *reinterpret_cast<const int*>(p + 4 * h);
     return v;
 }
 
@@ -206,14 +201,45 @@ __device__ __forceinline__ void chunk_store(int8_t* p, v4i v, int left, int vec)
 #pragma unroll
         for (int h = 0; h < 2; h++)
             if (left >= 8 * h + 8) *reinterpret_cast<v2i*>(p + 8 * h) = v2i{v[2 * h], v[2 * h + 1]};
-    } else if (vec == 4) {
+    } else {
 #pragma unroll
         for (int h = 0; h < 4; h++)
             if (left >= 4 * h + 4) *reinterpret_cast<int*>(p + 4 * h) = v[h];
-    } else {
+    }
+}
+
+// The thread and its lane, opaque: addresses made from them are computed where
+// they are used, not kept in registers across the requant (which spilled).
+__device__ __forceinline__ int gen_tid() {
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));
+    return tid;
+}
+__device__ __forceinline__ int gen_lane() { return gen_tid() & 63; }
+
+// Any channel count and address (vec 1): bytes, a lane per channel, so that an
+// access is whole rows of the block's channels: as many rows as fit 64 lanes
+// with each row's channels rounded up to a power of two.  (16 channels a lane,
+// as bytes or as unaligned vectors, took twice the time or more of a whole
+// launch: 1x1 256->131 @45 at 31 faces 47.5 us, now 22.9; 3x3 192->131
+// residual+BN @56 at 49 faces 251, 108.)  The block: `rows` of up to ROWS
+// pixels, `chans` of up to CW channels; v = get(row, channel) for a place of
+// the block, put(row, channel, v).
+template <int ROWS, int CW, typename G, typename P>
+__device__ __forceinline__ void row_bytes(long long rows, int chans, G get, P put) {
+    const int end = (int)(rows < ROWS ? rows : ROWS), w = chans < CW ? chans : CW;
+    constexpr int U = 4;                               // accesses in flight
+    if (end <= 0 || w <= 0) return;
+    const int sh = w > 1 ? 32 - __builtin_clz(w - 1) : 0;
+    const int lane = gen_lane(), step = 64 >> sh;
+    const int row0 = lane >> sh, ch = lane & ((1 << sh) - 1);
+    for (int r = 0; r < end; r += U * step) {
+        int8_t v[U];
 #pragma unroll
-        for (int e = 0; e < 16; e++)
-            if (e < left) p[e] = (int8_t)((uint32_t)v[e >> 2] >> (8 * (e & 3)));
+        for (int u = 0; u < U; u++) v[u] = get(min(r + u * step + row0, end - 1), min(ch, w - 1));
+#pragma unroll
+        for (int u = 0; u < U; u++)
+            if (r + u * step + row0 < end && ch < w) put(r + u * step + row0, ch, v[u]);
     }
 }
 
@@ -241,9 +267,10 @@ constexpr int GEN_LUT_BYTES = 64 * FF_LUT_PITCH;
 
 template <int NJ>
 __device__ __forceinline__ void gen_lut_load(const ConvArgs& a, const GenGeom& g, int n0, int j, v4i (&t)[4]) {
+    const int tid = gen_tid();
 #pragma unroll
     for (int k = 0; k < 4; k++) {
-        const int i = k * 256 + threadIdx.x;
+        const int i = k * 256 + tid;
         const int c = i >> 4, n = n0 + (c >> 5) * (NJ * 32) + j * 32 + (c & 31);
         typedef int v4i_any __attribute__((ext_vector_type(4), aligned(1)));
         t[k] = v4i{0, 0, 0, 0};
@@ -252,9 +279,10 @@ __device__ __forceinline__ void gen_lut_load(const ConvArgs& a, const GenGeom& g
 }
 
 __device__ __forceinline__ void gen_lut_store(const v4i (&t)[4], int8_t* lut) {
+    const int tid = gen_tid();
 #pragma unroll
     for (int k = 0; k < 4; k++) {
-        const int i = k * 256 + threadIdx.x;
+        const int i = k * 256 + tid;
         *reinterpret_cast<v4i*>(lut + (i >> 4) * FF_LUT_PITCH + (i & 15) * 16) = t[k];
     }
 }
@@ -268,40 +296,62 @@ __device__ __forceinline__ uint32_t pack_sat_i8(int a, int b, int c, int d) {
     return __builtin_amdgcn_perm(hi, lo, 0x05040100u);
 }
 
-// The wave's MI x NJ blocks at tile (m0 + wr, n0 + wc) to the staging tile
-// `stage` and X to memory.  prm: the tile's parameter rows.  RANGE and PRELU
+// The epilogue's three parts are separate functions, so that its five forms
+// (gen_requant) share the code of the other two: a small launch's epilogue runs
+// once, from code that is not in the instruction cache yet.
+
+// The residual of the wave's MI x NJ blocks at tile (m0, n0 + wc) -> its
+// staging tile
+template <int MI, int NJ>
+__device__ __forceinline__ void gen_residual(const ConvArgs& a, const GenGeom& g, long long m0, int n, int8_t* stage) {
+    constexpr int P = NJ * 32 + 16;                    // staging row pitch
+    constexpr int CH = NJ * 2, RPI = 64 / CH;          // 16-byte chunks per row, rows per chunk access
+    const int lane = gen_lane();
+    if (g.vec == 1) {
+        const int8_t* src = a.add_src + (size_t)m0 * g.cout + n;
+        row_bytes<MI * 32, NJ * 32>(a.M - m0, g.cout - n, [&](int row, int ch) { return src[row * g.cout + ch]; },
+                                    [&](int row, int ch, int8_t v) { stage[row * P + ch] = v; });
+    } else {
+        constexpr int U = 4;                           // chunks in flight
+        constexpr int N = MI * 32 / RPI;
+        auto fetch = [&](int vec) {
+#pragma unroll
+            for (int k0 = 0; k0 < N; k0 += U) {
+                v4i v[U];
+#pragma unroll
+                for (int u = 0; u < U && k0 + u < N; u++) {
+                    const int nc = n + (lane % CH) * 16;
+                    const long long m = m0 + lane / CH + (k0 + u) * RPI;
+                    v[u] = v4i{0, 0, 0, 0};
+                    if (m < a.M && nc < g.cout) v[u] = chunk_load(a.add_src + (size_t)m * g.cout + nc, g.cout - nc, vec);
+                }
+#pragma unroll
+                for (int u = 0; u < U && k0 + u < N; u++)
+                    *reinterpret_cast<v4i*>(stage + (lane / CH + (k0 + u) * RPI) * P + (lane % CH) * 16) = v[u];
+                asm volatile("" ::: "memory");
+            }
+        };
+        if (g.vec == 16) fetch(16);
+        else fetch(g.vec);
+    }
+    __builtin_amdgcn_wave_barrier();                   // (the wave's own tile: its LDS accesses run in order)
+}
+
+// The wave's blocks (channels wc.. of the tile) -> int8 in its staging tile,
+// which holds the residual.  prm: the tile's parameter rows.  RANGE and PRELU
 // as in wave_epi_i8 (0 / 1 with the flags read at run time: the general
 // form).  PIPE: a group's
 // parameters are read one group ahead of its arithmetic (not beside the BN
 // tables in flight: 128 registers keep four workgroups per CU).
 template <int MI, int NJ, int BN, int RANGE, int PRELU, bool PIPE>
-__device__ __forceinline__ void gen_epi_i8(const v16i (&acc)[MI][NJ], const ConvArgs& a, const GenGeom& g, long long m0,
-                                           int n0, int wc, int8_t* stage, const float* prm) {
+__device__ __forceinline__ void gen_requant(const v16i (&acc)[MI][NJ], const ConvArgs& a, int wc, int8_t* stage,
+                                            const float* prm) {
     typedef float v4f __attribute__((ext_vector_type(4)));
-    constexpr int P = NJ * 32 + 16;                    // staging row pitch
-    constexpr int CH = NJ * 2, RPI = 64 / CH;          // 16-byte chunks per row, rows per chunk access
+    constexpr int P = NJ * 32 + 16;
     const int lane = threadIdx.x & 63;
     const int lc = lane & 31, lh = lane >> 5;
     const bool add = RANGE != 2 && (a.flags & FFK_EPI_ADD), prelu = PRELU && (a.flags & FFK_EPI_PRELU);
     const bool insc = RANGE == 0 && (a.flags & FFK_EPI_INSCALE);
-    if (add) {
-        v4i v[MI * 32 / RPI];
-        auto fetch = [&](int vec) {
-#pragma unroll
-            for (int k = 0; k < MI * 32 / RPI; k++) {
-                const int n = n0 + wc + (lane % CH) * 16;
-                const long long m = m0 + lane / CH + k * RPI;
-                v[k] = v4i{0, 0, 0, 0};
-                if (m < a.M && n < g.cout) v[k] = chunk_load(a.add_src + (size_t)m * g.cout + n, g.cout - n, vec);
-            }
-        };
-        if (g.vec == 16) fetch(16);
-        else fetch(g.vec);
-#pragma unroll
-        for (int k = 0; k < MI * 32 / RPI; k++)
-            *reinterpret_cast<v4i*>(stage + (lane / CH + k * RPI) * P + (lane % CH) * 16) = v[k];
-        __builtin_amdgcn_wave_barrier();               // (the wave's own tile: its LDS accesses run in order)
-    }
     struct Prm { v4f ws, bias, inv, slope, adds; };
     auto params = [&](int t) {                         // of group t: channels (t/4)*32 + (t%4)*8 + lh*4 ..
         const float* pr = prm + wc + (t >> 2) * 32 + (t & 3) * 8 + lh * 4;
@@ -347,37 +397,59 @@ __device__ __forceinline__ void gen_epi_i8(const v16i (&acc)[MI][NJ], const Conv
         if (!PIPE && t + 1 < NJ * 4) nxt = params(t + 1);
     }
     __builtin_amdgcn_wave_barrier();
-    const bool x_even = (a.flags & FFK_OUT_X_EVEN) != 0;
-    if (!a.out) return;
+}
+
+// The wave's staging tile -> X, or X at its even pixels
+template <int MI, int NJ>
+__device__ __forceinline__ void gen_store_x(const ConvArgs& a, const GenGeom& g, long long m0, int n, const int8_t* stage) {
+    constexpr int P = NJ * 32 + 16, CH = NJ * 2, RPI = 64 / CH;
+    const int lane = gen_lane();
+    if (a.flags & FFK_OUT_X_EVEN) {
+        const unsigned hw = (unsigned)(g.hout * g.wout);
+#pragma unroll 1
+        for (int k = 0; k < MI * 32 / RPI; k++) {
+            const int row = lane / CH + k * RPI, ch = (lane % CH) * 16;
+            const long long m = m0 + row;
+            if (m >= a.M || n + ch >= g.cout) continue;
+            const unsigned bb = (unsigned)m / hw, rem = (unsigned)m - bb * hw;
+            const unsigned oh = rem / (unsigned)g.wout, ow = rem - oh * g.wout;
+            if ((oh | ow) & 1) continue;
+            const long long px = ((long long)bb * (g.hout / 2) + (oh >> 1)) * (g.wout / 2) + (ow >> 1);
+            int8_t* dst = a.out + (size_t)px * g.cout + n + ch;
+            if (g.vec > 1) chunk_store(dst, *reinterpret_cast<const v4i*>(stage + row * P + ch), g.cout - n - ch, g.vec);
+            else
+                for (int e = 0; e < min(16, g.cout - n - ch); e++) dst[e] = stage[row * P + ch + e];
+        }
+        return;
+    }
     auto flush = [&](int vec) {
 #pragma unroll
         for (int k = 0; k < MI * 32 / RPI; k++) {
-            const int row = lane / CH + k * RPI, ch = (lane % CH) * 16, n = n0 + wc + ch;
+            const int row = lane / CH + k * RPI, ch = (lane % CH) * 16;
             const long long m = m0 + row;
-            if (m >= a.M || n >= g.cout) continue;
-            const v4i v = *reinterpret_cast<const v4i*>(stage + row * P + ch);
-            long long px = m;
-            if (x_even) {
-                const int hw = g.hout * g.wout;
-                const int bb = (int)(m / hw);
-                const int rem = (int)(m - (long long)bb * hw);
-                const int oh = rem / g.wout, ow = rem - oh * g.wout;
-                if ((oh | ow) & 1) continue;
-                px = ((long long)bb * (g.hout / 2) + (oh >> 1)) * (g.wout / 2) + (ow >> 1);
-            }
-            chunk_store(a.out + (size_t)px * g.cout + n, v, g.cout - n, vec);
+            if (m >= a.M || n + ch >= g.cout) continue;
+            chunk_store(a.out + (size_t)m * g.cout + n + ch, *reinterpret_cast<const v4i*>(stage + row * P + ch),
+                        g.cout - n - ch, vec);
         }
     };
-    if (g.vec == 16) flush(16);
-    else flush(g.vec);
+    if (g.vec == 16) {
+        flush(16);
+    } else if (g.vec > 1) {
+        flush(g.vec);
+    } else {
+        int8_t* dst = a.out + (size_t)m0 * g.cout + n;
+        row_bytes<MI * 32, NJ * 32>(a.M - m0, g.cout - n, [&](int row, int ch) { return stage[row * P + ch]; },
+                                    [&](int row, int ch, int8_t v) { dst[row * g.cout + ch] = v; });
+    }
 }
 
 // BN(X) of the staging tile's j-th 32-channel block, through the round's
-// tables (those of this wave's column at `lut`)
+// tables (those of this wave's column at `lut`); the block is not read again
 template <int MI, int NJ>
 __device__ __forceinline__ void gen_bn_round(const ConvArgs& a, const GenGeom& g, long long m0, int n0, int j,
-                                             const int8_t* stage, const int8_t* lut) {
-    const int lane = threadIdx.x & 63;
+                                             int8_t* stage, const int8_t* lut) {
+    constexpr int P = NJ * 32 + 16;
+    const int lane = gen_lane();
     const int ch = (lane & 1) * 16, n = n0 + j * 32 + ch;
     auto flush = [&](int vec) {
 #pragma unroll
@@ -385,7 +457,8 @@ __device__ __forceinline__ void gen_bn_round(const ConvArgs& a, const GenGeom& g
         const int row = i * 32 + (lane >> 1);
         const long long m = m0 + row;
         if (m >= a.M || n >= g.cout) continue;
-        const v4i v = *reinterpret_cast<const v4i*>(stage + row * (NJ * 32 + 16) + j * 32 + ch);
+        v4i* s = reinterpret_cast<v4i*>(stage + row * P + j * 32 + ch);
+        const v4i v = *s;
         const int8_t* L = lut + ch * FF_LUT_PITCH + 128;
         v4i w;
 #pragma unroll
@@ -398,11 +471,21 @@ __device__ __forceinline__ void gen_bn_round(const ConvArgs& a, const GenGeom& g
             const uint32_t hi = __builtin_amdgcn_perm(b[3], b[2], 0x0c0c0400u);
             w[d] = (int)__builtin_amdgcn_perm(hi, lo, 0x05040100u);
         }
-        chunk_store(a.out_bn + (size_t)m * g.cout + n, w, g.cout - n, vec);
+        if (vec > 1) chunk_store(a.out_bn + (size_t)m * g.cout + n, w, g.cout - n, vec);
+        else *s = w;
     }
     };
-    if (g.vec == 16) flush(16);
-    else flush(g.vec);
+    if (g.vec == 16) {
+        flush(16);
+    } else if (g.vec > 1) {
+        flush(g.vec);
+    } else {
+        flush(1);
+        __builtin_amdgcn_wave_barrier();
+        int8_t* dst = a.out_bn + (size_t)m0 * g.cout + n0 + j * 32;
+        row_bytes<MI * 32, 32>(a.M - m0, g.cout - n0 - j * 32, [&](int row, int c) { return stage[row * P + j * 32 + c]; },
+                               [&](int row, int c, int8_t v) { dst[row * g.cout + c] = v; });
+    }
 }
 
 // All of it after the K loop: smem is the workgroup's LDS (the operands are
@@ -411,11 +494,18 @@ constexpr int gen_epi_bytes(int BM, int BN, bool LUT) {
     return 4 * gen_stage_bytes(BM / 64, BN / 64) + (LUT ? GEN_LUT_BYTES : 0);
 }
 
+// Workgroups per CU the registers have to allow: what each tile's K loop
+// needs (at 130 registers 24->256 5x5 @45 at 52 faces took 46.6 us, 39.4 at 124)
+constexpr int gen_occupancy(int BM, int BN, bool LUT, int RUN) {
+    const int blocks = BM / 64 * (BN / 64);
+    return blocks == 4 ? (RUN != 16 && LUT ? 3 : 4) : blocks == 2 ? 5 : 6;
+}
+
 template <int BM, int BN, bool LUT>
 __device__ __forceinline__ void gen_epilogue(const v16i (&acc)[BM / 64][BN / 64], const ConvArgs& a, const GenGeom& g,
                                              long long m0, int n0, int wr, int wc, int8_t* smem, const float* prm) {
     constexpr int MI = BM / 64, NJ = BN / 64;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     if (a.out_i32) {
 #pragma unroll
         for (int i = 0; i < MI; i++)
@@ -448,13 +538,15 @@ __device__ __forceinline__ void gen_epilogue(const v16i (&acc)[BM / 64][BN / 64]
     const bool pr = (f & FFK_EPI_PRELU) != 0;
     const bool rng = (f & FFK_EPI_IN_RANGE) && !(f & FFK_EPI_INSCALE) && (!pr || (f & FFK_EPI_PRELU_LE1));
     const bool fma = rng && (f & FFK_EPI_FMA_TAIL) && !(f & FFK_EPI_ADD);
-#define FF_GEN_EPI(RG, PR) gen_epi_i8<MI, NJ, BN, RG, PR, !LUT>(acc, a, g, m0 + wr, n0, wc, stage, prm)
+    if (f & FFK_EPI_ADD) gen_residual<MI, NJ>(a, g, m0 + wr, n0 + wc, stage);
+#define FF_GEN_EPI(RG, PR) gen_requant<MI, NJ, BN, RG, PR, !LUT>(acc, a, wc, stage, prm)
     if (!rng) FF_GEN_EPI(0, 1);
     else if (fma && pr) FF_GEN_EPI(2, 2);
     else if (fma) FF_GEN_EPI(2, 0);
     else if (pr) FF_GEN_EPI(1, 2);
     else FF_GEN_EPI(1, 0);
 #undef FF_GEN_EPI
+    if (a.out) gen_store_x<MI, NJ>(a, g, m0 + wr, n0 + wc, stage);
     if constexpr (LUT) {
 #pragma unroll
         for (int j = 0; j < NJ; j++) {
@@ -476,7 +568,7 @@ __device__ __forceinline__ void gen_epilogue(const v16i (&acc)[BM / 64][BN / 64]
 // operand per MAC: every staged A row serves BN output channels, every B row
 // BM output pixels.
 template <int RUN, int BM, int BN, bool LUT>
-__global__ __launch_bounds__(256, 3) void conv_generic_kernel(ConvArgs a, GenGeom g) {
+__global__ __launch_bounds__(256, gen_occupancy(BM, BN, LUT, RUN)) void conv_generic_kernel(ConvArgs a, GenGeom g) {
     constexpr int AR = BM / 64, BR = BN / 64;          // operand rows each thread stages
     constexpr int MI = BM / 64, NJ = BN / 64;          // 32x32 blocks per wave (2 x 2 waves)
     // one 64-byte K step per barrier pair (two or four steps' pieces staged
@@ -488,7 +580,7 @@ __global__ __launch_bounds__(256, 3) void conv_generic_kernel(ConvArgs a, GenGeo
     __shared__ __align__(16) float prm[GEN_NPRM * BN];
     int8_t* As = smem;
     int8_t* Bs = smem + BM * PITCH;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int tiles_n = (g.cout + BN - 1) / BN;
     // Workgroups go round-robin over the 8 XCDs: give each XCD a contiguous
     // run of tiles (N fastest), so the tiles that gather the same pixels
@@ -585,7 +677,7 @@ __global__ __launch_bounds__(256, 3) void conv_generic_kernel(ConvArgs a, GenGeo
 constexpr int GEN_NST = 2;
 
 template <int BM, int BN, bool LUT>
-__global__ __launch_bounds__(256, 4) void conv_generic_dma_kernel(ConvArgs a, GenGeom g) {
+__global__ __launch_bounds__(256, gen_occupancy(BM, BN, LUT, 16)) void conv_generic_dma_kernel(ConvArgs a, GenGeom g) {
     constexpr int MI = BM / 64, NJ = BN / 64;          // 32x32 blocks per wave (2 x 2 waves)
     constexpr int A_BYTES = BM * 64, B_BYTES = BN * 64, STAGE = A_BYTES + B_BYTES;
     constexpr int A_LD = A_BYTES / (256 * 16), B_LD = B_BYTES / (256 * 16);

@@ -36,7 +36,16 @@ def test_generic_bn_table_at_any_address(gpu_lib, oracle, cin, cout, k, pad, H, 
     _check(gpu_lib, oracle, cin, cout, k, pad, H, B, (0, 0, 0), lut_offset)
 
 
-def _check(lib, oracle, cin, cout, k, pad, H, B, offsets, lut_offset=0):
+# X at its even pixels only, beside BN at all of them, for every vector width,
+# 64- and 128-row tiles and the register-staged operands
+@pytest.mark.parametrize("cin,cout,k,pad,H,B", [(32, 33, 3, 1, 10, 2), (16, 131, 1, 0, 12, 3), (24, 36, 3, 1, 10, 2),
+                                                (32, 136, 3, 1, 12, 2), (16, 67, 1, 0, 58, 12), (7, 5, 3, 1, 10, 2)])
+@pytest.mark.parametrize("offsets", [(0, 0, 0), (3, 4, 1)])
+def test_generic_x_even(gpu_lib, oracle, cin, cout, k, pad, H, B, offsets):
+    _check(gpu_lib, oracle, cin, cout, k, pad, H, B, offsets, x_even=True)
+
+
+def _check(lib, oracle, cin, cout, k, pad, H, B, offsets, lut_offset=0, x_even=False):
     r = rng(4100 + cin + cout * 3 + H)
     ho = H + 2 * pad - k + 1
     x = r.integers(-128, 128, size=(B, H, H, cin), dtype=np.int8)
@@ -65,13 +74,15 @@ def _check(lib, oracle, cin, cout, k, pad, H, B, offsets, lut_offset=0):
     d.in_, d.w, d.params, d.bn_lut = dx.ptr, dw.ptr, dp.ptr, dl.ptr + lut_offset
     d.add_src, d.out, d.out_bn = da.ptr + offsets[2], do.ptr + offsets[0], db.ptr + offsets[1]
     d.flags = fa.FFK_EPI_BIAS | fa.FFK_EPI_PRELU | fa.FFK_EPI_ADD | fa.FFK_EPI_BN
+    if x_even:
+        d.flags |= fa.FFK_OUT_X_EVEN
     assert lib.ffk_conv_variant(C.byref(d)) == b"generic"
     check(lib, lib.ffk_conv(C.byref(d), None))
     check(lib, lib.ffk_stream_sync(None))
     exp = oracle.fused_epilogue(oracle.conv_i32(x, w, 1, pad), ws=ws, bias=bias, prelu=slope, add_src=add,
                                 add_scale_pc=adds, inv_pc=inv)
     exp_bn = oracle.bn_prelu_requant(exp, in_scale_pc=bsin, bn_scale=bns, bn_offset=bno, inv_pc=binv)
-    for dev, off, e in ((do, offsets[0], exp), (db, offsets[1], exp_bn)):
+    for dev, off, e in ((do, offsets[0], exp[:, ::2, ::2] if x_even else exp), (db, offsets[1], exp_bn)):
         got = dev.get(np.int8, (n + 64,))
-        assert np.array_equal(got[off:off + n].reshape(e.shape), e)
-        assert (got[:off] == 0x5a).all() and (got[off + n:] == 0x5a).all()
+        assert np.array_equal(got[off:off + e.size].reshape(e.shape), e)
+        assert (got[:off] == 0x5a).all() and (got[off + e.size:] == 0x5a).all()
